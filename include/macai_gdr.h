@@ -51,7 +51,7 @@
 extern "C" {
 #endif
 
-#define MACAI_GDR_ABI_VERSION 13
+#define MACAI_GDR_ABI_VERSION 14
 
 /* dtype codes (the rule takes F32 and BF16; the producers also F16) */
 #define MACAI_GDR_F32 0
@@ -205,6 +205,17 @@ int macai_gdr_conv_bwd(const void* x, const float* w, const void* dq, const void
                        float* dwp, float* dw, int64_t B, int64_t T, int64_t C, int64_t KD, int64_t DK, int64_t REP,
                        int64_t DV, int32_t dtype, int32_t vdtype, void* stream);
 
+/* The two entry points above with the taps in their own type (wdtype: F32, BF16 or F16), so that a layer whose weights
+ * train in 2 bytes makes no conversions around them: the forward reads w [C, 4] in wdtype and, with taps non-NULL,
+ * writes its float32 copy there (what the backward takes); the backward writes dw [C, 4] in wdtype (rounded from the
+ * float32 sum). */
+int macai_gdr_conv_fwd_typed(const void* x, const void* w, int32_t wdtype, float* taps, void* q, void* k, void* v,
+                             int64_t B, int64_t T, int64_t C, int64_t KD, int64_t DK, int64_t REP, int64_t DV,
+                             int32_t dtype, int32_t vdtype, void* stream);
+int macai_gdr_conv_bwd_typed(const void* x, const float* w, const void* dq, const void* dk, const void* dv, void* dx,
+                             float* dwp, void* dw, int32_t wdtype, int64_t B, int64_t T, int64_t C, int64_t KD,
+                             int64_t DK, int64_t REP, int64_t DV, int32_t dtype, int32_t vdtype, void* stream);
+
 /* float32 elements of the conv backward's dw partials for a shape. */
 int64_t macai_gdr_conv_partials(int64_t B, int64_t T, int64_t C);
 
@@ -221,6 +232,22 @@ int macai_gdr_gates_fwd(const void* b, const void* a, const float* A_log, const 
 int macai_gdr_gates_bwd(const void* b, const void* a, const float* A_log, const float* dt_bias, const float* dbeta,
                         const float* dg, void* db, void* da, float* dA_log, float* ddt_bias, int64_t n, int64_t H,
                         int32_t dtype, void* stream);
+
+/* The two entry points above with A_log and dt_bias in their own types (codes atype, dtype_bias: F32, BF16 or F16).  The
+ * forward writes their float32 copies [2, H] to params when it is non-NULL (what the backward takes).  The backward
+ * always writes dA_log and ddt_bias, in those types: its one pass forms its workgroups' sums in part, double
+ * [macai_gdr_gates_partials(n, H)] scratch, and a second launch adds them in a fixed order, where macai_gdr_gates_bwd
+ * without scratch runs a pass of one workgroup a head. */
+int macai_gdr_gates_fwd_typed(const void* b, const void* a, const void* A_log, int32_t atype, const void* dt_bias,
+                              int32_t dtype_bias, float* params, float* beta, float* g, int64_t n, int64_t H,
+                              int32_t dtype, void* stream);
+int macai_gdr_gates_bwd_typed(const void* b, const void* a, const float* A_log, const float* dt_bias,
+                              const float* dbeta, const float* dg, void* db, void* da, double* part, void* dA_log,
+                              int32_t atype, void* ddt_bias, int32_t dtype_bias, int64_t n, int64_t H, int32_t dtype,
+                              void* stream);
+
+/* Doubles of macai_gdr_gates_bwd_typed's scratch for n elements over H heads. */
+int64_t macai_gdr_gates_partials(int64_t n, int64_t H);
 
 /* ---- measurement ---- */
 

@@ -6,16 +6,13 @@
 //   (The reference's layer/_conv.py:1-24 and layer/_gates.py:1-13 state the same functions.)
 //
 // The convolution is an HBM stream: every input and output byte crosses once (the 3-row halos come again through L2).
-// Work goes by 16-byte channel vectors (8 bf16 / f16 or 4 fp32 channels).  The forward gives a lane one vector over 8
-// consecutive time steps, all 11 input rows loaded at once, a wave 64 consecutive vectors (conv_fwd_kernel).  The
-// backward needs du = dy silu'(u) at 3 rows past each output row and shares it between neighbouring outputs, so it runs
-// on LDS tiles: a workgroup stages x (64 + 6 rows: a 3-row halo each side, by asynchronous global -> LDS copies) and the
-// upstream gradient (67 rows, a key head's copies summed) of 8 vectors, forms du for the tile in LDS (float32) and
-// gathers dx from du's windows, every lane in parallel over time: one writer an element.  The taps' gradient is a
-// per-tile correlation of du with x from the same LDS tiles, reduced over the tile's rows in a fixed order (lane pairs,
-// then the four waves through LDS); sum_columns_kernel adds the tiles' partials in tile order: deterministic.
-// The gates are one pass each way, an element a lane; A_log's and dt_bias's gradients take one
-// workgroup a head, rows split over its waves and summed in a fixed tree.
+// A lane owns a channel vector over consecutive time steps, all its input rows loaded at once, a wave 64 consecutive
+// vectors: 4 channels over 8 steps in the forward (conv_fwd_kernel), over 16 or 8 in the backward (conv_bwd_kernel),
+// which forms du = dy silu'(u) for its steps and the 3 after them in registers, dx from du's
+// windows (one writer an element) and the taps' gradient's sums over its steps; a tile of 64 rows adds its waves' sums
+// in order through LDS, sum_columns_kernel the tiles' partials in tile order: deterministic.
+// The gates are one pass each way, an element a lane; the backward's also forms its workgroup's sums of A_log's and
+// dt_bias's gradients, which a second launch adds in a fixed tree.
 #include <hip/hip_runtime.h>
 
 #include "gdr_abi.h"
@@ -25,10 +22,7 @@ namespace gdr {
 
 typedef _Float16 f16;
 
-// ---- 16-byte vectors of 2- or 4-byte elements, as floats -----------------------------------------------------------
-template <typename T> struct V16 {
-  static constexpr int N = 16 / (int)sizeof(T);   // elements in 16 bytes
-};
+// ---- vectors of 2- or 4-byte elements, as floats ------------------------------------------------------------------
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 
 // The 32-bit words of N values of T (N * sizeof(T) a multiple of 4), and back.
@@ -40,9 +34,8 @@ __device__ __forceinline__ void to_words(const float (&x)[N], unsigned (&wd)[N *
   } else {
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) {
-      const unsigned short lo = __builtin_bit_cast(unsigned short, (T)x[2 * i]);
-      const unsigned short hi = __builtin_bit_cast(unsigned short, (T)x[2 * i + 1]);
-      wd[i] = (unsigned)lo | ((unsigned)hi << 16);
+      typedef T T2 __attribute__((ext_vector_type(2)));
+      wd[i] = __builtin_bit_cast(unsigned, T2{(T)x[2 * i], (T)x[2 * i + 1]});   // one packed conversion
     }
   }
 }
@@ -73,77 +66,65 @@ __device__ __forceinline__ void store_as(T* p, const float (&x)[N]) {
     *reinterpret_cast<u32x4_t*>(q + s) = u32x4_t{wd[s], wd[s + 1], wd[s + 2], wd[s + 3]};
   if constexpr (NW % 4 == 2) *reinterpret_cast<u32x2_t*>(q + NW - 2) = u32x2_t{wd[NW - 2], wd[NW - 1]};
 }
-// N values of T from memory as floats, with the same access widths.
+// N values of T from memory as floats, in one load of N * sizeof(T) bytes.
 template <typename T, int N>
 __device__ __forceinline__ void load_as(const T* p, float (&x)[N]) {
   constexpr int NW = N * (int)sizeof(T) / 4;
-  static_assert(NW % 2 == 0, "whole 8-byte pieces");
+  typedef unsigned words_t __attribute__((ext_vector_type(NW)));
+  const words_t r = *reinterpret_cast<const words_t*>(p);
   unsigned wd[NW];
-  const unsigned* q = reinterpret_cast<const unsigned*>(p);
 #pragma unroll
-  for (int s = 0; s + 4 <= NW; s += 4) {
-    const u32x4_t r = *reinterpret_cast<const u32x4_t*>(q + s);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) wd[s + i] = r[i];
-  }
-  if constexpr (NW % 4 == 2) {
-    const u32x2_t r = *reinterpret_cast<const u32x2_t*>(q + NW - 2);
-    wd[NW - 2] = r[0];
-    wd[NW - 1] = r[1];
-  }
+  for (int i = 0; i < NW; ++i) wd[i] = r[i];
   from_words<T, N>(wd, x);
-}
-
-// The V16<T>::N values of T in the 16 bytes `raw`, as floats.
-template <typename T>
-__device__ __forceinline__ void unpack(const u32x4_t& raw, float (&x)[V16<T>::N]) {
-  const unsigned wd[4] = {raw[0], raw[1], raw[2], raw[3]};
-  from_words<T, V16<T>::N>(wd, x);
 }
 
 // ---- the convolution path ----------------------------------------------------------------------------------------
 constexpr int CV_TAPS = 4;
-constexpr int CV_ROWS = 64;       // output time steps a tile
-constexpr int CV_VECS = 8;        // 16-byte channel vectors a tile row
-constexpr int CV_THREADS = 256;   // 32 row groups x 8 vectors; a lane computes rows rg and rg + 32
+constexpr int CV_ROWS = 64;       // time steps a tile of the backward
 constexpr int CV_HALO = CV_TAPS - 1;
 
 struct ConvArgs {
   const void* x;                  // [B, T, C] in T
-  const float* w;                 // [C, 4] float32 taps
+  const void* w;                  // [C, 4] taps, dtype code wt
+  float* taps;                    // forward: the taps' float32 copy for the backward, or null
   void *q, *k, *v;                // forward outputs: q, k [B, T, KD * REP] in T, v [B, T, C - 2 KD] in TV
   const void *dq, *dk, *dv;       // backward inputs, same layouts
   void* dx;                       // [B, T, C] in T
   float* part;                    // [B * ntiles, C * 4] per-tile taps' gradient, or null
   int B, T, C, KD, DK, REP, ntiles;
+  int wt;
 };
 
 // Where a 16-byte channel vector lives among the outputs: q, k (key heads, each written REP times: REP = 1 keeps key
 // heads only) or v.  A vector never straddles a head (head widths are multiples of the vector).
 struct Dest {
   int which;                      // 0 q, 1 k, 2 v
-  size_t pitch;                   // row pitch of the destination (elements)
-  size_t col;                     // the vector's first column there (copy 0)
+  unsigned pitch;                 // row pitch of the destination (elements)
+  unsigned col;                     // the vector's first column there (copy 0)
   __device__ Dest(int c, int KD, int DK, int REP, int C) {
     if (c < 2 * KD) {
       which = c < KD ? 0 : 1;
       const int cc = c - which * KD;
-      pitch = (size_t)KD * REP;
-      col = (size_t)(cc / DK) * REP * DK + cc % DK;
+      pitch = (unsigned)(KD * REP);
+      col = (unsigned)((cc / DK) * REP * DK + cc % DK);
     } else {
       which = 2;
-      pitch = (size_t)(C - 2 * KD);
-      col = (size_t)(c - 2 * KD);
+      pitch = (unsigned)(C - 2 * KD);
+      col = (unsigned)(c - 2 * KD);
     }
   }
 };
 
-// The tile's taps, tap-major: tw[j][i] = w[c + i, j] for the lane's N channels.
+// The tile's taps, tap-major: tw[j][i] = w[c + i, j] for the lane's N channels; w in the type of code wt (uniform).
 template <int N>
-__device__ __forceinline__ void tile_taps(const float* w, int c, float (&tw)[CV_TAPS][N]) {
+__device__ __forceinline__ void tile_taps(const void* w, int wt, int c, float (&tw)[CV_TAPS][N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const f4 r = *reinterpret_cast<const f4*>(w + (size_t)(c + i) * CV_TAPS);
+    float r[CV_TAPS];
+    const size_t at = (size_t)(c + i) * CV_TAPS;
+    if (wt == MACAI_GDR_F32) load_as<float, CV_TAPS>((const float*)w + at, r);
+    else if (wt == MACAI_GDR_BF16) load_as<bf16, CV_TAPS>((const bf16*)w + at, r);
+    else load_as<f16, CV_TAPS>((const f16*)w + at, r);
 #pragma unroll
     for (int j = 0; j < CV_TAPS; ++j) tw[j][i] = r[j];
   }
@@ -163,81 +144,82 @@ __device__ __forceinline__ float tap_dot(const float (&tw)[CV_TAPS][N], int i, f
     return fmaf(tw[0][i], w0, fmaf(tw[1][i], w1, fmaf(tw[2][i], w2, tw[3][i] * w3)));
   }
 }
+// 1 / d for d >= 1 (or NaN): the hardware reciprocal (1 ulp) and one Newton step, r + r (1 - d r), which rounds as the
+// division does but for rare ties (d held finite, so that an overflowed exponential still gives 0).  The division took a
+// fifth of the backward's instructions; the results' errors against float64 are the same to four digits.
+__device__ __forceinline__ float recip(float d) {
+  d = fminf(d, 3.0e38f);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
 template <bool EXACT>
 __device__ __forceinline__ float logistic(float u) {
   if constexpr (EXACT) return 1.0f / (1.0f + expf(-u));
-  else return __frcp_rn(1.0f + __expf(-u));
+  else return recip(1.0f + __expf(-u));
 }
 // u sigmoid(u) with one rounding after the exponential for float32 inputs (a division, not u times a rounded
 // reciprocal, whose two roundings put the float32 output past twice PyTorch's silu error)
 template <bool EXACT>
 __device__ __forceinline__ float silu(float u) {
   if constexpr (EXACT) return u / (1.0f + expf(-u));
-  else return u * __frcp_rn(1.0f + __expf(-u));
+  else return u * recip(1.0f + __expf(-u));
 }
 
-// Stage rows [t_lo, t_lo + NROWS) x the tile's CV_VECS vectors of x (batch row b) into LDS by asynchronous 16-byte
-// copies (global -> LDS, no registers), all of a thread's issued back to back; units outside [0, T) or past the
-// channels are zeroed by LDS stores instead.  Unit u = row * CV_VECS + vector.  The caller waits (wait_copies) and
-// synchronises before reading.
-template <typename T, int NROWS>
-__device__ __forceinline__ void stage_x(u32x4_t* dst, const T* xb, int t_lo, int c0, int T_, int C) {
-  constexpr int VE = V16<T>::N;
-  constexpr int UNITS = NROWS * CV_VECS, PER = (UNITS + CV_THREADS - 1) / CV_THREADS;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int u = threadIdx.x + i * CV_THREADS;
-    if (u < UNITS) {
-      const int row = u / CV_VECS, c = c0 + (u % CV_VECS) * VE, t = t_lo + row;
-      if (t >= 0 && t < T_ && c < C)
-        __builtin_amdgcn_global_load_lds((const void*)(xb + (size_t)t * C + c),
-                                         (__attribute__((address_space(3))) void*)(dst + u - threadIdx.x % 64), 16,
-                                         0, 0);
-      else
-        dst[u] = u32x4_t{0u, 0u, 0u, 0u};
-    }
-  }
-}
-__device__ __forceinline__ void wait_copies() { __builtin_amdgcn_s_waitcnt(0); }
-
-// The forward needs no staging: a lane owns one 16-byte channel vector over CV_FWD_STEPS consecutive time steps and
-// issues the loads of all its CV_FWD_STEPS + 3 input rows at once (the 3 halo rows come again through L2), then forms
-// each output from them.  A wave spans 64 consecutive vectors (1 KB of a bf16 row), a workgroup four consecutive time
-// blocks.  Measured at config 1's widths this ran at the box's mixed read/write rate, ahead of LDS-staged tiles (whose
-// staging and barrier put each tile's loads and stores in separate phases).
+constexpr int CV_VE = 4;          // channels a lane
+// The forward needs no staging: a lane owns 4 channels over 8 consecutive time steps and issues the loads of all its 11
+// input rows at once (the 3 halo rows come again through L2), then forms each output from them.  A wave spans 64
+// consecutive vectors of one block of steps (a wave-uniform start: row addresses are scalar and the ends of the row
+// cost the other waves nothing), a workgroup four consecutive blocks.  Bound by its bytes once the chip is full: at
+// B = 4, T = 1024, C = 6144 in bf16 (101 MB, 18 us at the box's copy rate) 23.0 us, at C = 8192 and T = 2048 (268 MB)
+// 49.9 us, 5.4 TB/s.  Lanes of 8 channels (16-byte loads) took 25.0 and 51.5 us (half the waves, twice the registers),
+// 4 or 16 steps 22.9-23.7 and 50.9-52.8; with a correctly rounded division in silu 28.8 and 61 us.
 constexpr int CV_FWD_STEPS = 8;
 template <typename T, typename TV>
 __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
-  constexpr int VE = V16<T>::N;
+  constexpr int VE = CV_VE;
   constexpr bool EXACT = sizeof(T) == 4;
-  constexpr int NR = CV_FWD_STEPS + CV_HALO;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  constexpr int S = CV_FWD_STEPS, NR = S + CV_HALO;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = (blockIdx.x * 64 + lane) * VE;
-  const int t0 = (blockIdx.y * 4 + wave) * CV_FWD_STEPS, b = blockIdx.z;
-  if (c >= a.C || t0 >= a.T) return;
-  const T* xb = (const T*)a.x + (size_t)b * a.T * a.C + c;
-  u32x4_t raw[NR];                                    // x[t0 - 3 + i], zero outside the sequence
+  const int t0 = (blockIdx.y * 4 + wave) * S, b = blockIdx.z, Tn = a.T;   // t0: uniform in a wave
+  if (c >= a.C || t0 >= Tn) return;
+  typedef unsigned wordx_t __attribute__((ext_vector_type(VE * sizeof(T) / 4)));
+  const int row0 = b * Tn;                 // B T C < 2^31
+  wordx_t xr[NR];                          // x[t0 - 3 + i], zero outside the sequence (see conv_bwd_kernel)
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
     const int t = t0 - CV_HALO + i;
-    raw[i] = (t >= 0 && t < a.T) ? *reinterpret_cast<const u32x4_t*>(xb + (size_t)t * a.C) : u32x4_t{0u, 0u, 0u, 0u};
+    const size_t row = (unsigned)(row0 + (t < 0 ? 0 : t < Tn ? t : Tn - 1));
+    xr[i] = *reinterpret_cast<const wordx_t*>((const T*)a.x + row * a.C + c);
   }
   float tw[CV_TAPS][VE];
-  tile_taps<VE>(a.w, c, tw);
-  const Dest d(c, a.KD, a.DK, a.REP, a.C);
+  tile_taps<VE>(a.w, a.wt, c, tw);
+  if (a.taps && t0 == 0 && b == 0)         // one wave a channel range
 #pragma unroll
-  for (int s = 0; s < CV_FWD_STEPS; ++s) {
-    const int t = t0 + s;
-    if (t >= a.T) break;
-    float w0[VE], w1[VE], w2[VE], w3[VE];             // x[t - 3] .. x[t]
-    unpack<T>(raw[s], w0);
-    unpack<T>(raw[s + 1], w1);
-    unpack<T>(raw[s + 2], w2);
-    unpack<T>(raw[s + 3], w3);
+    for (int e = 0; e < VE; ++e)
+      *reinterpret_cast<f4*>(a.taps + (size_t)(c + e) * CV_TAPS) = f4{tw[0][e], tw[1][e], tw[2][e], tw[3][e]};
+  if (t0 < CV_HALO || t0 + S > Tn)
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      if (t0 - CV_HALO + i < 0 || t0 - CV_HALO + i >= Tn) xr[i] = wordx_t{};
+  const Dest d(c, a.KD, a.DK, a.REP, a.C);
+  float xw[CV_TAPS][VE];                   // x[t - 3 .. t], oldest first
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+#pragma unroll
+    for (int j = 0; j + 1 < CV_TAPS; ++j)
+#pragma unroll
+      for (int e = 0; e < VE; ++e) xw[j][e] = xw[j + 1][e];
+    unsigned wd[VE * sizeof(T) / 4];
+#pragma unroll
+    for (int e = 0; e < (int)(VE * sizeof(T) / 4); ++e) wd[e] = xr[i][e];
+    from_words<T, VE>(wd, xw[3]);
+    const int t = t0 + i - CV_HALO;
+    if (i < CV_HALO || t >= Tn) continue;
     float y[VE];
 #pragma unroll
-    for (int i = 0; i < VE; ++i) y[i] = silu<EXACT>(tap_dot<EXACT, VE>(tw, i, w0[i], w1[i], w2[i], w3[i]));
-    const size_t row = (size_t)b * a.T + t;
+    for (int e = 0; e < VE; ++e) y[e] = silu<EXACT>(tap_dot<EXACT, VE>(tw, e, xw[0][e], xw[1][e], xw[2][e], xw[3][e]));
+    const size_t row = (unsigned)(row0 + t);
     if (d.which == 2) {
       store_as<TV, VE>((TV*)a.v + row * d.pitch + d.col, y);
     } else {
@@ -247,162 +229,190 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
   }
 }
 
-// The backward of a tile of 64 output rows t0 .. t0 + 63 (dx there, and the tile's share of the taps' gradient):
-//   x staged for t0 - 3 .. t0 + 66, the upstream gradient dy (q's and k's copies summed in copy order) for
-//   t0 .. t0 + 66, then du = dy s (1 + u (1 - s)), s = sigmoid(u), in place (0 past the end), then
+// The backward, like the forward, streams: a lane owns 4 channels over S consecutive time steps t0 .. t0 + S - 1 and
+// issues all its loads at once -- x[t0 - 3 .. t0 + S + 2] and the upstream gradient dy[t0 .. t0 + S + 2] (q's and k's
+// copies summed in copy order) -- then walks the rows with everything in registers:
+//   du[t] = dy s (1 + u (1 - s)), s = sigmoid(u)   (0 past the end), for its S rows and the 3 after them,
 //   dx[t] = w0 du[t + 3] + w1 du[t + 2] + w2 du[t + 1] + w3 du[t],
-//   part[tile][c, j] = sum over the tile's t of du[t] x[t - 3 + j].
+//   part[tile][c, j] = sum over the tile's t of du[t] x[t - 3 + j], in double.
+// A workgroup is one tile of 64 rows: 64 / S waves, a time block each, over the same 64 vectors, whose sums meet in
+// LDS in wave order (deterministic).  S + 3 rows of du for S of dx: at S = 16 the recomputed rows cost a fifth of the
+// activations.  4-byte x takes twice the registers a row, so it runs S = 8 (all of a lane's loads in flight at 2 waves
+// a SIMD).  Its 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27 us at the box's copy rate and its VALU work is about
+// as long.  Measured there: 36 us, 41 with the taps' gradient (its double sums), against 45 and 65 for the form that
+// staged tiles of x and dy in LDS (three barriers, every row through LDS as float32 twice); at C = 8192, T = 2048 82
+// and 97 against 114 and 154.  S = 8 for bf16 was as fast without the taps' gradient and 14 us slower with it; three
+// waves a SIMD spills.
+template <typename T> constexpr int conv_bwd_steps() { return sizeof(T) == 4 ? 8 : 16; }
 template <typename T, typename TV, bool TAPS>
-__global__ void __launch_bounds__(CV_THREADS) conv_bwd_tile_kernel(ConvArgs a) {
-  constexpr int VE = V16<T>::N;
+__global__ void __launch_bounds__(64 * (CV_ROWS / conv_bwd_steps<T>()), 2) conv_bwd_kernel(ConvArgs a) {
+  constexpr int VE = CV_VE, S = conv_bwd_steps<T>(), NWAVE = CV_ROWS / S;
   constexpr bool EXACT = sizeof(T) == 4;
-  constexpr int XR = CV_ROWS + 2 * CV_HALO;          // x rows t0 - 3 .. t0 + 66
-  constexpr int DR = CV_ROWS + CV_HALO;              // du rows t0 .. t0 + 66
-  __shared__ u32x4_t xs[XR * CV_VECS];
-  __shared__ float du[DR * CV_VECS * VE];            // [row][vector][element]
-  __shared__ double red[4][32][TAPS ? VE : 1];       // the taps' gradient: one row of partials a wave
-  const int c0 = blockIdx.x * CV_VECS * VE, t0 = blockIdx.y * CV_ROWS, b = blockIdx.z;
-  const T* xb = (const T*)a.x + (size_t)b * a.T * a.C;
-  stage_x<T, XR>(xs, xb, t0 - CV_HALO, c0, a.T, a.C);
-  // dy for rows t0 .. t0 + 66 (zero past the end or past the channels): every unit's first-copy load is issued
-  // before any is used (a thread's units keep its vector, so they share one destination map)
-  {
-    constexpr int UNITS = DR * CV_VECS, PER = (UNITS + CV_THREADS - 1) / CV_THREADS;
-    const int vec = threadIdx.x % CV_VECS, c = c0 + vec * VE;
-    const Dest d(c < a.C ? c : 0, a.KD, a.DK, a.REP, a.C);
-    const T* qk = (const T*)(d.which == 0 ? a.dq : a.dk);
-    float g[PER][VE];
-    bool live[PER];
+  constexpr int XR = S + 2 * CV_HALO, DR = S + CV_HALO;
+  __shared__ double red[TAPS ? NWAVE : 1][TAPS ? VE : 1][64];   // one tap's sums: a row a wave
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cl = (blockIdx.x * 64 + lane) * VE;
+  const bool on = cl < a.C;                // lanes past the channels repeat the last vector and store nothing
+  const int c = on ? cl : a.C - VE;
+  const int t0 = blockIdx.y * CV_ROWS + wave * S, b = blockIdx.z, Tn = a.T;   // t0: uniform in a wave
+  const int row0 = b * Tn;                 // B T C < 2^31
+  typedef unsigned wordx_t __attribute__((ext_vector_type(VE * sizeof(T) / 4)));
+  typedef unsigned wordv_t __attribute__((ext_vector_type(VE * sizeof(TV) / 4)));
+  double acc[CV_TAPS][VE];
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int u = threadIdx.x + i * CV_THREADS, t = t0 + u / CV_VECS;
-      live[i] = u < UNITS && t < a.T && c < a.C;
-      const size_t r = (size_t)b * a.T + (live[i] ? t : 0);
-      if (d.which == 2) load_as<TV, VE>((const TV*)a.dv + r * d.pitch + d.col, g[i]);
-      else load_as<T, VE>(qk + r * d.pitch + d.col, g[i]);
-    }
-    if (d.which != 2)
-      for (int rep = 1; rep < a.REP; ++rep)   // the other copies of a repeated key head, added in copy order
+  for (int j = 0; j < CV_TAPS; ++j)
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-          const int t = t0 + (threadIdx.x + i * CV_THREADS) / CV_VECS;
-          const size_t r = (size_t)b * a.T + (live[i] ? t : 0);
+    for (int i = 0; i < VE; ++i) acc[j][i] = 0.0;
+  if (t0 < Tn) {                           // the waves past the end only join the sums
+    // rows outside the sequence read a row inside it, so that every load is unconditional; the waves that have such
+    // rows (their first or last block) zero them after
+    const bool edge = t0 < CV_HALO || t0 + DR > Tn;
+    auto row_of = [&](int t) { return (size_t)(unsigned)(row0 + (t < 0 ? 0 : t < Tn ? t : Tn - 1)); };
+    wordx_t xr[XR];                        // x[t0 - 3 + i]
+#pragma unroll
+    for (int i = 0; i < XR; ++i)
+      xr[i] = *reinterpret_cast<const wordx_t*>((const T*)a.x + row_of(t0 - CV_HALO + i) * a.C + c);
+    const Dest d(c, a.KD, a.DK, a.REP, a.C);
+    float g[DR][VE];                       // dy[t0 + i]
+    if (d.which == 2) {
+      const TV* src = (const TV*)a.dv + d.col;
+      wordv_t r[DR];
+#pragma unroll
+      for (int i = 0; i < DR; ++i) r[i] = *reinterpret_cast<const wordv_t*>(src + row_of(t0 + i) * d.pitch);
+#pragma unroll
+      for (int i = 0; i < DR; ++i) {
+        unsigned wd[VE * sizeof(TV) / 4];
+#pragma unroll
+        for (int e = 0; e < (int)(VE * sizeof(TV) / 4); ++e) wd[e] = r[i][e];
+        from_words<TV, VE>(wd, g[i]);
+      }
+    } else {
+      const T* src = (const T*)(d.which == 0 ? a.dq : a.dk) + d.col;
+      for (int rep = 0; rep < a.REP; ++rep, src += a.DK) {   // a repeated key head's copies, added in copy order
+        wordx_t r[DR];
+#pragma unroll
+        for (int i = 0; i < DR; ++i) r[i] = *reinterpret_cast<const wordx_t*>(src + row_of(t0 + i) * d.pitch);
+#pragma unroll
+        for (int i = 0; i < DR; ++i) {
+          unsigned wd[VE * sizeof(T) / 4];
           float h[VE];
-          load_as<T, VE>(qk + r * d.pitch + d.col + (size_t)rep * a.DK, h);
 #pragma unroll
-          for (int e = 0; e < VE; ++e) g[i][e] += h[e];
+          for (int e = 0; e < (int)(VE * sizeof(T) / 4); ++e) wd[e] = r[i][e];
+          from_words<T, VE>(wd, h);
+#pragma unroll
+          for (int e = 0; e < VE; ++e) g[i][e] = rep ? g[i][e] + h[e] : h[e];
         }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int u = threadIdx.x + i * CV_THREADS;
-      if (u < UNITS)
-#pragma unroll
-        for (int e = 0; e < VE; ++e) du[u * VE + e] = live[i] ? g[i][e] : 0.f;
+      }
     }
-  }
-  wait_copies();
-  __syncthreads();
-  float tw[CV_TAPS][VE];
-  {
-    const int vec = threadIdx.x % CV_VECS, c = c0 + vec * VE;
-    if (c < a.C) tile_taps<VE>(a.w, c, tw);
-    else
+    if (edge) {
 #pragma unroll
-      for (int j = 0; j < CV_TAPS; ++j)
+      for (int i = 0; i < XR; ++i)
+        if (t0 - CV_HALO + i < 0 || t0 - CV_HALO + i >= Tn) xr[i] = wordx_t{};
 #pragma unroll
-        for (int i = 0; i < VE; ++i) tw[j][i] = 0.f;
-  }
-  // du in place: unit u's row sees x rows row .. row + 3 (t - 3 .. t); the lanes of a unit keep their vector, so tw
-  // is the lane's own taps
-  for (int u = threadIdx.x; u < DR * CV_VECS; u += CV_THREADS) {
-    const int row = u / CV_VECS, vec = u % CV_VECS;
-    float w0[VE], w1[VE], w2[VE], w3[VE];
-    unpack<T>(xs[(row + 0) * CV_VECS + vec], w0);
-    unpack<T>(xs[(row + 1) * CV_VECS + vec], w1);
-    unpack<T>(xs[(row + 2) * CV_VECS + vec], w2);
-    unpack<T>(xs[(row + 3) * CV_VECS + vec], w3);
+      for (int i = 0; i < DR; ++i)
+        if (t0 + i >= Tn)
 #pragma unroll
-    for (int i = 0; i < VE; ++i) {
-      const float uu = tap_dot<EXACT, VE>(tw, i, w0[i], w1[i], w2[i], w3[i]);
-      const float s = logistic<EXACT>(uu);
-      du[u * VE + i] *= s * (1.0f + uu * (1.0f - s));   // dy was staged there (0 past the end)
+          for (int e = 0; e < VE; ++e) g[i][e] = 0.f;
     }
-  }
-  __syncthreads();
-
-  // dx for the lane's rows rg, rg + 32
-  {
-    const int vec = threadIdx.x % CV_VECS, rg = threadIdx.x / CV_VECS, c = c0 + vec * VE;
-    if (c < a.C) {
-      T* dxb = (T*)a.dx + (size_t)b * a.T * a.C + c;
+    float tw[CV_TAPS][VE];
+    tile_taps<VE>(a.w, a.wt, c, tw);
+    T* dxb = (T*)a.dx + (size_t)row0 * a.C + c;
+    float xw[CV_TAPS][VE], dw[CV_TAPS][VE];   // x[t - 3 .. t] and du[t - 3 .. t], oldest first
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int r = rg + 32 * h, t = t0 + r;
-        if (t >= a.T) break;
+    for (int j = 1; j < CV_TAPS; ++j) {       // x[t0 - 3 .. t0 - 1] in places 1 .. 3
+      unsigned wd[VE * sizeof(T) / 4];
+#pragma unroll
+      for (int e = 0; e < (int)(VE * sizeof(T) / 4); ++e) wd[e] = xr[j - 1][e];
+      from_words<T, VE>(wd, xw[j]);
+    }
+#pragma unroll
+    for (int s = 0; s < DR; ++s) {
+#pragma unroll
+      for (int j = 0; j + 1 < CV_TAPS; ++j)
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+          xw[j][i] = xw[j + 1][i];
+          if (s) dw[j][i] = dw[j + 1][i];
+        }
+      unsigned wd[VE * sizeof(T) / 4];
+#pragma unroll
+      for (int e = 0; e < (int)(VE * sizeof(T) / 4); ++e) wd[e] = xr[s + CV_HALO][e];
+      from_words<T, VE>(wd, xw[3]);
+#pragma unroll
+      for (int i = 0; i < VE; ++i) {
+        const float uu = tap_dot<EXACT, VE>(tw, i, xw[0][i], xw[1][i], xw[2][i], xw[3][i]);
+        const float sg = logistic<EXACT>(uu);
+        dw[3][i] = g[s][i] * (sg * (1.0f + uu * (1.0f - sg)));
+      }
+      if (TAPS && s < S)
+#pragma unroll
+        for (int i = 0; i < VE; ++i) {
+          const double dd = (double)dw[3][i];
+#pragma unroll
+          for (int j = 0; j < CV_TAPS; ++j) acc[j][i] = fma(dd, (double)xw[j][i], acc[j][i]);
+        }
+      if (s >= CV_HALO && on && t0 + s - CV_HALO < Tn) {
         float o[VE];
-        const float* d0 = du + ((r + 3) * CV_VECS + vec) * VE;   // du[t + 3]
-        const float* d1 = du + ((r + 2) * CV_VECS + vec) * VE;
-        const float* d2 = du + ((r + 1) * CV_VECS + vec) * VE;
-        const float* d3 = du + ((r + 0) * CV_VECS + vec) * VE;   // du[t]
 #pragma unroll
-        for (int i = 0; i < VE; ++i) o[i] = tap_dot<EXACT, VE>(tw, i, d0[i], d1[i], d2[i], d3[i]);
-        store_as<T, VE>(dxb + (size_t)t * a.C, o);
+        for (int i = 0; i < VE; ++i) o[i] = tap_dot<EXACT, VE>(tw, i, dw[3][i], dw[2][i], dw[1][i], dw[0][i]);
+        store_as<T, VE>(dxb + (size_t)(t0 + s - CV_HALO) * a.C, o);
       }
     }
   }
   if constexpr (TAPS) {
-    // combo = (vector, tap) = lane % 32; part = thread / 32 sums rows 8 part .. 8 part + 7 in double
-    const int combo = threadIdx.x % 32, part = threadIdx.x / 32, vec = combo % CV_VECS, j = combo / CV_VECS;
-    double acc[VE];
+    // tap by tap: every wave's sums into LDS, then wave w adds channel i = w's over the waves in order
+    float* out = a.part + (size_t)(b * a.ntiles + blockIdx.y) * a.C * CV_TAPS;
 #pragma unroll
-    for (int i = 0; i < VE; ++i) acc[i] = 0.0;
+    for (int j = 0; j < CV_TAPS; ++j) {
+      if (j) __syncthreads();              // the previous tap's sums are read
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int r = 8 * part + s;                     // x[t - 3 + j] is staged row r + j
-      float xv[VE];
-      unpack<T>(xs[(r + j) * CV_VECS + vec], xv);
-      const float* dd = du + (r * CV_VECS + vec) * VE;
+      for (int i = 0; i < VE; ++i) red[wave][i][lane] = acc[j][i];
+      __syncthreads();
+      if (wave < VE && on) {
+        double s = red[0][wave][lane];
 #pragma unroll
-      for (int i = 0; i < VE; ++i) acc[i] = fma((double)dd[i], (double)xv[i], acc[i]);
-    }
-    // parts 2w and 2w + 1 are lanes l and l + 32 of wave w: add them, then the four waves in order through LDS
-#pragma unroll
-    for (int i = 0; i < VE; ++i) acc[i] += __shfl_xor(acc[i], 32, 64);
-    const int w = threadIdx.x / 64;
-    if ((threadIdx.x & 63) < 32)
-#pragma unroll
-      for (int i = 0; i < VE; ++i) red[w][combo][i] = acc[i];
-    __syncthreads();
-    if (threadIdx.x < 32) {
-      const int c = c0 + vec * VE;
-      if (c < a.C) {
-        float* out = a.part + (size_t)(b * a.ntiles + blockIdx.y) * a.C * CV_TAPS;
-#pragma unroll
-        for (int i = 0; i < VE; ++i)
-          out[(size_t)(c + i) * CV_TAPS + j] =
-              (float)(((red[0][combo][i] + red[1][combo][i]) + red[2][combo][i]) + red[3][combo][i]);
+        for (int w = 1; w < NWAVE; ++w) s += red[w][wave][lane];
+        out[(size_t)(c + wave) * CV_TAPS + j] = (float)s;
       }
     }
   }
 }
 
-// out[i] = the sum over rows p = 0 .. P - 1 of in[p * n + i], in row order, in double, rounded once: the fixed-order
-// second stage of the taps' gradient.  A lane an output; each row's loads for a group of eight rows are in flight
-// together.
-__global__ void __launch_bounds__(256) sum_columns_kernel(const float* in, float* out, int P, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+// x at element i of an array in the type of code t (uniform), and back.
+__device__ __forceinline__ void store_code(void* p, int t, size_t i, float x) {
+  if (t == MACAI_GDR_F32) ((float*)p)[i] = x;
+  else if (t == MACAI_GDR_BF16) ((bf16*)p)[i] = (bf16)x;
+  else ((f16*)p)[i] = (f16)x;
+}
+__device__ __forceinline__ float load_code(const void* p, int t, size_t i) {
+  if (t == MACAI_GDR_F32) return ((const float*)p)[i];
+  if (t == MACAI_GDR_BF16) return (float)((const bf16*)p)[i];
+  return (float)((const f16*)p)[i];
+}
+
+// out[i] = the sum over rows p = 0 .. P - 1 of in[p * n + i], in double, rounded to float32 and then to the type of code
+// ot: the fixed-order second stage of the taps' gradient.  A workgroup takes 64 outputs; each of its waves sums a quarter of the rows in row order, eight
+// rows' loads in flight together, and the quarters add in order.
+__global__ void __launch_bounds__(256) sum_columns_kernel(const float* in, void* out, int ot, int P, int n) {
+  __shared__ double quarter[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+  const int per = (P + 3) / 4, hi = min(P, (w + 1) * per);
   double s = 0.0;
-  int p = 0;
-  for (; p + 8 <= P; p += 8) {
-    float v[8];
+  if (i < n) {
+    int p = w * per;
+    for (; p + 8 <= hi; p += 8) {
+      float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = in[(size_t)(p + e) * n + i];
+      for (int e = 0; e < 8; ++e) v[e] = in[(size_t)(p + e) * n + i];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s += (double)v[e];
+      for (int e = 0; e < 8; ++e) s += (double)v[e];
+    }
+    for (; p < hi; ++p) s += (double)in[(size_t)p * n + i];
   }
-  for (; p < P; ++p) s += (double)in[(size_t)p * n + i];
-  out[i] = (float)s;
+  quarter[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && i < n)
+    store_code(out, ot, i, (float)(((quarter[0][lane] + quarter[1][lane]) + quarter[2][lane]) + quarter[3][lane]));
 }
 
 // ---- the gates -----------------------------------------------------------------------------------------------------
@@ -415,41 +425,113 @@ __device__ __forceinline__ double softplus_t20(double x) { return x > 20.0 ? x :
 __device__ __forceinline__ double softplus_t20_grad(double x) { return x > 20.0 ? 1.0 : 1.0 / (1.0 + exp(-x)); }
 
 // The gates move under a megabyte per layer, so they are bound by latency, not bandwidth: one element a lane, so
-// that a layer's elements spread over every lane of the chip and each lane runs one exponential chain.
+// that a layer's elements spread over every lane of the chip and each lane runs one exponential chain.  A_log and
+// dt_bias are read in the types of codes pt[0], pt[1]; with `params` non-null the first lanes write their float32
+// copies ([2, H]) there.
 constexpr int GATE_THREADS = 256;
+struct GateParams {
+  const void *alog, *dtb;
+  int ta, td;                                // dtype codes
+  __device__ __forceinline__ float a(int h) const { return load_code(alog, ta, h); }
+  __device__ __forceinline__ float d(int h) const { return load_code(dtb, td, h); }
+};
 template <typename T>
-__global__ void __launch_bounds__(GATE_THREADS) gates_fwd_kernel(const T* b, const T* a, const float* alog,
-                                                                 const float* dtb, float* beta, float* g, int64_t n,
-                                                                 int H) {
+__global__ void __launch_bounds__(GATE_THREADS) gates_fwd_kernel(const T* b, const T* a, GateParams p, float* params,
+                                                                 float* beta, float* g, int64_t n, int H) {
   const int64_t i = (int64_t)blockIdx.x * GATE_THREADS + threadIdx.x;
   if (i >= n) return;
   const int head = (int)(i % H);             // heads run fastest: element i is head i mod H
-  const double rate = -exp((double)alog[head]);
+  const float alog = p.a(head), dtb = p.d(head);
+  if (params && i < H) {                     // n is a multiple of H
+    params[i] = alog;
+    params[H + i] = dtb;
+  }
+  const double rate = -exp((double)alog);
   beta[i] = (float)(1.0 / (1.0 + exp(-(double)(float)b[i])));
-  g[i] = (float)(rate * softplus_t20((double)(float)a[i] + (double)dtb[head]));
+  g[i] = (float)(rate * softplus_t20((double)(float)a[i] + (double)dtb));
 }
 
-template <typename T>
+// db = dbeta s (1 - s), s = sigmoid(b); da = dg (-exp(A_log)) softplus'(a + dt_bias).  PARTS: also each workgroup's
+// sums, per head, of the parameters' gradients' terms (dA_log: dg g; ddt_bias: da before its rounding), in double, to
+// part[workgroup][2][H].  A workgroup's elements go by whole rows of H heads: thread i of it takes head i % H of row
+// i / H and then every rpp-th row (rpp = 256 / H rows at once; heads past 256 in further passes), its own sums in row
+// order, and the rpp sums of a head add in order through LDS: deterministic.  gates_params_kernel adds the workgroups'
+// in order.  Bound by the chain of double exponentials, so it is spread over every CU: at B T = 4096, H = 16 in bf16
+// 6.0 us with the sums and 3.8 for gates_params_kernel, where this pass without them (3.5) and one of one workgroup a
+// head (14.8: two exponentials and a logarithm an element on H CUs) took 18.3.
+template <typename T, bool PARTS>
 __global__ void __launch_bounds__(GATE_THREADS) gates_bwd_kernel(const T* b, const T* a, const float* alog,
                                                                  const float* dtb, const float* dbeta,
-                                                                 const float* dg, T* db, T* da, int64_t n, int H) {
-  const int64_t i = (int64_t)blockIdx.x * GATE_THREADS + threadIdx.x;
-  if (i >= n) return;
-  const int head = (int)(i % H);
-  const double rate = -exp((double)alog[head]);
-  const double sig = 1.0 / (1.0 + exp(-(double)(float)b[i]));
-  db[i] = (T)(float)((double)dbeta[i] * (sig - sig * sig));          // d sigmoid = s (1 - s)
-  da[i] = (T)(float)((double)dg[i] * rate * softplus_t20_grad((double)(float)a[i] + (double)dtb[head]));
+                                                                 const float* dg, T* db, T* da, double* part,
+                                                                 int64_t rows, int H, int per) {
+  __shared__ double red[PARTS ? 2 : 1][PARTS ? GATE_THREADS : 1];
+  const int64_t r0 = (int64_t)blockIdx.x * per, r1 = r0 + per < rows ? r0 + per : rows;
+  const int rpp = H < GATE_THREADS ? GATE_THREADS / H : 1;   // rows at once
+  const int sub = H < GATE_THREADS ? threadIdx.x / H : 0;
+  for (int h0 = 0; h0 < H; h0 += GATE_THREADS) {
+    const int h = H < GATE_THREADS ? threadIdx.x % H : h0 + threadIdx.x;
+    double s_a = 0.0, s_d = 0.0;
+    if (sub < rpp && h < H) {
+      const double rate = -exp((double)alog[h]), bias = (double)dtb[h];
+      for (int64_t r = r0 + sub; r < r1; r += rpp) {
+        const int64_t i = r * H + h;
+        const double sig = 1.0 / (1.0 + exp(-(double)(float)b[i]));
+        db[i] = (T)(float)((double)dbeta[i] * (sig - sig * sig));          // d sigmoid = s (1 - s)
+        const double x = (double)(float)a[i] + bias, gr = (double)dg[i] * rate, dx = gr * softplus_t20_grad(x);
+        da[i] = (T)(float)dx;
+        if (PARTS) {
+          s_a = fma(gr, softplus_t20(x), s_a);
+          s_d += dx;
+        }
+      }
+    }
+    if constexpr (PARTS) {
+      if (h0) __syncthreads();               // the previous heads' sums are read
+      red[0][threadIdx.x] = s_a;
+      red[1][threadIdx.x] = s_d;
+      __syncthreads();
+      if (sub == 0 && h < H) {
+        for (int k = 1; k < rpp; ++k) {
+          s_a += red[0][k * H + h];
+          s_d += red[1][k * H + h];
+        }
+        double* out = part + (size_t)blockIdx.x * 2 * H;
+        out[h] = s_a;
+        out[H + h] = s_d;
+      }
+    }
+  }
 }
 
-// dA_log[h] = sum over rows of dg g and ddt[h] = sum over rows of dg (-exp(A_log)) softplus'(a + dt_bias): one
-// workgroup a head; thread i takes rows i, i + 256, ... in order, then a wave sums its lanes by a fixed butterfly and
-// the four waves add in order.  Deterministic.  Terms and sums in double, rounded once: a head's rows of dg carry both
-// signs, so the sums can cancel.
+// dA_log[h] and ddt_bias[h]: the workgroups' sums of gates_bwd_kernel added in double, rounded to float32 and then to
+// the gradients' types.  A wave a head: lane l adds workgroups l, l + 64, ... in order, then the lanes add by a fixed
+// butterfly.
+__global__ void __launch_bounds__(64) gates_params_kernel(const double* part, void* dA, void* ddt, int ta, int td,
+                                                          int groups, int H) {
+  const int h = blockIdx.x;
+  double s_a = 0.0, s_d = 0.0;
+  for (int w = threadIdx.x; w < groups; w += 64) {
+    s_a += part[(size_t)w * 2 * H + h];
+    s_d += part[(size_t)w * 2 * H + H + h];
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    s_a += __shfl_xor(s_a, off, 64);
+    s_d += __shfl_xor(s_d, off, 64);
+  }
+  if (threadIdx.x == 0) {
+    store_code(dA, ta, h, (float)s_a);
+    store_code(ddt, td, h, (float)s_d);
+  }
+}
+
+// The parameters' gradients for callers without scratch: one workgroup a head; thread i takes rows i, i + 256, ... in
+// order, then a wave sums its lanes by a fixed butterfly and the four waves add in order.  Deterministic.  Terms and
+// sums in double, rounded once: a head's rows of dg carry both signs, so the sums can cancel.
 template <typename T>
-__global__ void __launch_bounds__(256) gates_params_kernel(const T* a, const float* alog, const float* dtb,
-                                                           const float* dg, float* dA, float* ddt, int64_t rows,
-                                                           int H) {
+__global__ void __launch_bounds__(256) gates_params_direct_kernel(const T* a, const float* alog, const float* dtb,
+                                                                  const float* dg, float* dA, float* ddt, int64_t rows,
+                                                                  int H) {
   const int h = blockIdx.x;
   const double rate = -exp((double)alog[h]), bias = (double)dtb[h];
   double s_a = 0.0, s_d = 0.0;
@@ -504,13 +586,15 @@ int check_conv(const char* what, int64_t B, int64_t T, int64_t C, int64_t KD, in
   return MACAI_GDR_OK;
 }
 
-int64_t conv_tiles(int64_t T) { return (T + CV_ROWS - 1) / CV_ROWS; }
-
-// the launch grid of the conv kernels for element size es: channel tiles, time tiles, batch rows
-dim3 conv_grid(int64_t B, int64_t T, int64_t C, int es) {
-  const int64_t per = (int64_t)CV_VECS * (16 / es);
-  return dim3((unsigned)((C + per - 1) / per), (unsigned)conv_tiles(T), (unsigned)B);
+// The gates' backward's workgroups for `rows` rows of H heads, `per` rows each: one pass of rows a workgroup (an element
+// a lane) up to 512 workgroups, then as many passes as keep to that (the second stage adds the workgroups' sums).
+int64_t gate_groups(int64_t rows, int64_t H, int64_t* per) {
+  const int64_t rpp = H < GATE_THREADS ? GATE_THREADS / H : 1;
+  *per = rpp * ((rows + rpp * 512 - 1) / (rpp * 512));
+  return (rows + *per - 1) / *per;
 }
+
+int64_t conv_tiles(int64_t T) { return (T + CV_ROWS - 1) / CV_ROWS; }
 
 }  // namespace
 
@@ -531,17 +615,24 @@ extern "C" {
 
 int macai_gdr_conv_fwd(const void* x, const float* w, void* q, void* k, void* v, int64_t B, int64_t T, int64_t C,
                        int64_t KD, int64_t DK, int64_t REP, int64_t DV, int32_t dtype, int32_t vdtype, void* stream) {
+  return macai_gdr_conv_fwd_typed(x, w, MACAI_GDR_F32, nullptr, q, k, v, B, T, C, KD, DK, REP, DV, dtype, vdtype, stream);
+}
+
+int macai_gdr_conv_fwd_typed(const void* x, const void* w, int32_t wdtype, float* taps, void* q, void* k, void* v,
+                             int64_t B, int64_t T, int64_t C, int64_t KD, int64_t DK, int64_t REP, int64_t DV,
+                             int32_t dtype, int32_t vdtype, void* stream) {
   const char* what = "macai_gdr_conv_fwd";
+  if (wdtype < MACAI_GDR_F32 || wdtype > MACAI_GDR_F16)
+    return fail(MACAI_GDR_EUNSUP, "%s: dtype codes must be F32, BF16 or F16", what);
   if (int rc = check_conv(what, B, T, C, KD, DK, REP, DV, dtype, vdtype)) return rc;
   if (!x || !w || !q || !k || !v) return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
-  const void* ps[] = {x, w, q, k, v};
+  const void* ps[] = {x, w, taps, q, k, v};
   for (const void* p : ps)
     if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
-  ConvArgs a{x, w, q, k, v, nullptr, nullptr, nullptr, nullptr, nullptr, (int)B, (int)T, (int)C, (int)KD, (int)DK,
-             (int)REP, (int)conv_tiles(T)};
+  ConvArgs a{x, w, taps, q, k, v, nullptr, nullptr, nullptr, nullptr, nullptr, (int)B, (int)T, (int)C, (int)KD, (int)DK,
+             (int)REP, (int)conv_tiles(T), wdtype};
   hipStream_t st = (hipStream_t)stream;
-  const int es = dtype == MACAI_GDR_F32 ? 4 : 2;
-  const dim3 grid((unsigned)((C / (16 / es) + 63) / 64), (unsigned)((T + 4 * CV_FWD_STEPS - 1) / (4 * CV_FWD_STEPS)),
+  const dim3 grid((unsigned)((C + 64 * CV_VE - 1) / (64 * CV_VE)), (unsigned)((T + 4 * CV_FWD_STEPS - 1) / (4 * CV_FWD_STEPS)),
                   (unsigned)B);
   DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_fwd_kernel<PT, PV>), grid, dim3(256), 0, st, a)))
   return launched(what);
@@ -550,7 +641,16 @@ int macai_gdr_conv_fwd(const void* x, const float* w, void* q, void* k, void* v,
 int macai_gdr_conv_bwd(const void* x, const float* w, const void* dq, const void* dk, const void* dv, void* dx,
                        float* dwp, float* dw, int64_t B, int64_t T, int64_t C, int64_t KD, int64_t DK, int64_t REP,
                        int64_t DV, int32_t dtype, int32_t vdtype, void* stream) {
+  return macai_gdr_conv_bwd_typed(x, w, dq, dk, dv, dx, dwp, dw, MACAI_GDR_F32, B, T, C, KD, DK, REP, DV, dtype, vdtype,
+                                  stream);
+}
+
+int macai_gdr_conv_bwd_typed(const void* x, const float* w, const void* dq, const void* dk, const void* dv, void* dx,
+                             float* dwp, void* dw, int32_t wdtype, int64_t B, int64_t T, int64_t C, int64_t KD,
+                             int64_t DK, int64_t REP, int64_t DV, int32_t dtype, int32_t vdtype, void* stream) {
   const char* what = "macai_gdr_conv_bwd";
+  if (wdtype < MACAI_GDR_F32 || wdtype > MACAI_GDR_F16)
+    return fail(MACAI_GDR_EUNSUP, "%s: dtype codes must be F32, BF16 or F16", what);
   if (int rc = check_conv(what, B, T, C, KD, DK, REP, DV, dtype, vdtype)) return rc;
   if (!x || !w || !dq || !dk || !dv || !dx) return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
   if (!dwp != !dw) return fail(MACAI_GDR_EINVAL, "%s: dwp and dw go together (both or neither)", what);
@@ -558,22 +658,22 @@ int macai_gdr_conv_bwd(const void* x, const float* w, const void* dq, const void
   for (const void* p : ps)
     if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
   const int ntiles = (int)conv_tiles(T);
-  ConvArgs a{x, w, nullptr, nullptr, nullptr, dq, dk, dv, dx, dwp, (int)B, (int)T, (int)C, (int)KD, (int)DK,
-             (int)REP, ntiles};
+  ConvArgs a{x, w, nullptr, nullptr, nullptr, nullptr, dq, dk, dv, dx, dwp, (int)B, (int)T, (int)C, (int)KD, (int)DK,
+             (int)REP, ntiles, MACAI_GDR_F32};
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid = conv_grid(B, T, C, dtype == MACAI_GDR_F32 ? 4 : 2);
+  // 64 vectors of CV_VE channels by a tile of CV_ROWS steps; a wave a block of conv_bwd_steps of them
+  const dim3 grid((unsigned)((C + 64 * CV_VE - 1) / (64 * CV_VE)), (unsigned)ntiles, (unsigned)B);
+  const dim3 block(64 * (CV_ROWS / (dtype == MACAI_GDR_F32 ? conv_bwd_steps<float>() : conv_bwd_steps<bf16>())));
   if (dwp) {
-    DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_tile_kernel<PT, PV, true>), grid,
-                                                              dim3(CV_THREADS), 0, st, a)))
+    DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_kernel<PT, PV, true>), grid, block, 0, st, a)))
   } else {
-    DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_tile_kernel<PT, PV, false>), grid,
-                                                              dim3(CV_THREADS), 0, st, a)))
+    DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_kernel<PT, PV, false>), grid, block, 0, st, a)))
   }
   if (int rc = launched(what)) return rc;
   if (dw) {
     const int n = (int)(C * CV_TAPS);
-    hipLaunchKernelGGL(sum_columns_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dwp, dw,
-                       (int)(B * ntiles), n);
+    hipLaunchKernelGGL(sum_columns_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, dwp, dw,
+                       wdtype, (int)(B * ntiles), n);
     return launched(what);
   }
   return MACAI_GDR_OK;
@@ -581,19 +681,60 @@ int macai_gdr_conv_bwd(const void* x, const float* w, const void* dq, const void
 
 int64_t macai_gdr_conv_partials(int64_t B, int64_t T, int64_t C) { return B * conv_tiles(T) * C * CV_TAPS; }
 
-int macai_gdr_gates_fwd(const void* b, const void* a, const float* A_log, const float* dt_bias, float* beta, float* g,
-                        int64_t n, int64_t H, int32_t dtype, void* stream) {
+static bool param_type_ok(int32_t t) { return t >= MACAI_GDR_F32 && t <= MACAI_GDR_F16; }
+
+int macai_gdr_gates_fwd_typed(const void* b, const void* a, const void* A_log, int32_t atype, const void* dt_bias,
+                              int32_t dtype_bias, float* params, float* beta, float* g, int64_t n, int64_t H,
+                              int32_t dtype, void* stream) {
   const char* what = "macai_gdr_gates_fwd";
   if (n < 1 || H < 1 || n % H) return fail(MACAI_GDR_EINVAL, "%s: need n >= 1 a multiple of H >= 1", what);
-  if (dtype < MACAI_GDR_F32 || dtype > MACAI_GDR_F16) return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
+  if (dtype < MACAI_GDR_F32 || dtype > MACAI_GDR_F16 || !param_type_ok(atype) || !param_type_ok(dtype_bias))
+    return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
   if (!b || !a || !A_log || !dt_bias || !beta || !g) return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
   const void* ps[] = {b, a, beta, g};
   for (const void* p : ps)
     if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)((n + GATE_THREADS - 1) / GATE_THREADS));
+  const GateParams gp{A_log, dt_bias, atype, dtype_bias};
   DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_fwd_kernel<PT>), grid, dim3(GATE_THREADS), 0, st, (const PT*)b,
-                                        (const PT*)a, A_log, dt_bias, beta, g, n, (int)H))
+                                        (const PT*)a, gp, params, beta, g, n, (int)H))
+  return launched(what);
+}
+
+int macai_gdr_gates_fwd(const void* b, const void* a, const float* A_log, const float* dt_bias, float* beta, float* g,
+                        int64_t n, int64_t H, int32_t dtype, void* stream) {
+  return macai_gdr_gates_fwd_typed(b, a, A_log, MACAI_GDR_F32, dt_bias, MACAI_GDR_F32, nullptr, beta, g, n, H, dtype,
+                                   stream);
+}
+
+int64_t macai_gdr_gates_partials(int64_t n, int64_t H) {
+  if (n < 1 || H < 1 || n % H) return 0;
+  int64_t per;
+  return gate_groups(n / H, H, &per) * 2 * H;
+}
+
+static int gates_bwd(const char* what, const void* b, const void* a, const float* A_log, const float* dt_bias,
+                     const float* dbeta, const float* dg, void* db, void* da, double* part, int64_t n, int64_t H,
+                     int32_t dtype, void* stream) {
+  if (n < 1 || H < 1 || n % H) return fail(MACAI_GDR_EINVAL, "%s: need n >= 1 a multiple of H >= 1", what);
+  if (dtype < MACAI_GDR_F32 || dtype > MACAI_GDR_F16) return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
+  if (!b || !a || !A_log || !dt_bias || !dbeta || !dg || !db || !da)
+    return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
+  const void* ps[] = {b, a, dbeta, dg, db, da};
+  for (const void* p : ps)
+    if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
+  int64_t per;
+  const int64_t rows = n / H, groups = gate_groups(rows, H, &per);
+  hipStream_t st = (hipStream_t)stream;
+  const dim3 grid((unsigned)groups), block(GATE_THREADS);
+  if (part) {
+    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_kernel<PT, true>), grid, block, 0, st, (const PT*)b, (const PT*)a,
+                                          A_log, dt_bias, dbeta, dg, (PT*)db, (PT*)da, part, rows, (int)H, (int)per))
+  } else {
+    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_kernel<PT, false>), grid, block, 0, st, (const PT*)b, (const PT*)a,
+                                          A_log, dt_bias, dbeta, dg, (PT*)db, (PT*)da, part, rows, (int)H, (int)per))
+  }
   return launched(what);
 }
 
@@ -601,25 +742,29 @@ int macai_gdr_gates_bwd(const void* b, const void* a, const float* A_log, const 
                         const float* dg, void* db, void* da, float* dA_log, float* ddt_bias, int64_t n, int64_t H,
                         int32_t dtype, void* stream) {
   const char* what = "macai_gdr_gates_bwd";
-  if (n < 1 || H < 1 || n % H) return fail(MACAI_GDR_EINVAL, "%s: need n >= 1 a multiple of H >= 1", what);
-  if (dtype < MACAI_GDR_F32 || dtype > MACAI_GDR_F16) return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
-  if (!b || !a || !A_log || !dt_bias || !dbeta || !dg || !db || !da)
-    return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
   if (!dA_log != !ddt_bias) return fail(MACAI_GDR_EINVAL, "%s: dA_log and ddt_bias go together", what);
-  const void* ps[] = {b, a, dbeta, dg, db, da};
-  for (const void* p : ps)
-    if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)((n + GATE_THREADS - 1) / GATE_THREADS));
-  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_kernel<PT>), grid, dim3(GATE_THREADS), 0, st, (const PT*)b,
-                                        (const PT*)a, A_log, dt_bias, dbeta, dg, (PT*)db, (PT*)da, n, (int)H))
-  if (int rc = launched(what)) return rc;
-  if (dA_log) {
-    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_params_kernel<PT>), dim3((unsigned)H), dim3(256), 0, st,
-                                          (const PT*)a, A_log, dt_bias, dg, dA_log, ddt_bias, n / H, (int)H))
-    return launched(what);
-  }
-  return MACAI_GDR_OK;
+  if (int rc = gates_bwd(what, b, a, A_log, dt_bias, dbeta, dg, db, da, nullptr, n, H, dtype, stream)) return rc;
+  if (!dA_log) return MACAI_GDR_OK;
+  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_params_direct_kernel<PT>), dim3((unsigned)H), dim3(256), 0,
+                                        (hipStream_t)stream, (const PT*)a, A_log, dt_bias, dg, dA_log, ddt_bias, n / H,
+                                        (int)H))
+  return launched(what);
+}
+
+int macai_gdr_gates_bwd_typed(const void* b, const void* a, const float* A_log, const float* dt_bias,
+                              const float* dbeta, const float* dg, void* db, void* da, double* part, void* dA_log,
+                              int32_t atype, void* ddt_bias, int32_t dtype_bias, int64_t n, int64_t H, int32_t dtype,
+                              void* stream) {
+  const char* what = "macai_gdr_gates_bwd";
+  if (!part || !dA_log || !ddt_bias) return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
+  if (!param_type_ok(atype) || !param_type_ok(dtype_bias)) return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
+  if (((uintptr_t)part & 7u) != 0) return fail(MACAI_GDR_EINVAL, "%s: the partial sums must be 8-byte aligned", what);
+  if (int rc = gates_bwd(what, b, a, A_log, dt_bias, dbeta, dg, db, da, part, n, H, dtype, stream)) return rc;
+  int64_t per;
+  const int64_t groups = gate_groups(n / H, H, &per);
+  hipLaunchKernelGGL(gates_params_kernel, dim3((unsigned)H), dim3(64), 0, (hipStream_t)stream, part, dA_log, ddt_bias,
+                     atype, dtype_bias, (int)groups, (int)H);
+  return launched(what);
 }
 
 }  // extern "C"

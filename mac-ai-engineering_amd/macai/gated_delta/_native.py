@@ -16,7 +16,7 @@ BF16_F32 = 3                          # MACAI_GDR_BF16_F32: bf16 tensors, float3
 OK, EINVAL, EUNSUP, ELAUNCH = 0, 1, 2, 3
 STORE_STATES, NO_OUTPUT = 1, 8
 NOALLOC_SCRATCH_BYTES = 128 << 20     # MACAI_GDR_NOALLOC_SCRATCH_BYTES
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 _p, _i64, _i32, _f = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_float
 # name -> argument types (the order of include/macai_gdr.h)
@@ -32,9 +32,14 @@ SIGNATURES = {
     "macai_gdr_group_sum": [_p] * 2 + [_i64] * 5 + [_i32, _p],
     "macai_gdr_conv_fwd": [_p] * 5 + [_i64] * 7 + [_i32, _i32, _p],
     "macai_gdr_conv_bwd": [_p] * 8 + [_i64] * 7 + [_i32, _i32, _p],
+    "macai_gdr_conv_fwd_typed": [_p] * 2 + [_i32] + [_p] * 4 + [_i64] * 7 + [_i32, _i32, _p],
+    "macai_gdr_conv_bwd_typed": [_p] * 8 + [_i32] + [_i64] * 7 + [_i32, _i32, _p],
     "macai_gdr_conv_partials": [_i64] * 3,
     "macai_gdr_gates_fwd": [_p] * 6 + [_i64] * 2 + [_i32, _p],
     "macai_gdr_gates_bwd": [_p] * 10 + [_i64] * 2 + [_i32, _p],
+    "macai_gdr_gates_fwd_typed": [_p] * 3 + [_i32, _p, _i32] + [_p] * 3 + [_i64] * 2 + [_i32, _p],
+    "macai_gdr_gates_bwd_typed": [_p] * 10 + [_i32, _p, _i32] + [_i64] * 2 + [_i32, _p],
+    "macai_gdr_gates_partials": [_i64] * 2,
     "macai_gdr_forward": [_p] * 9 + [_i64] * 7 + [_i32, _i32, _f, _i32, _p, _i64, _p],
     "macai_gdr_forward_workspace": [_i64] * 5 + [_i32, _i64],
     "macai_gdr_forward_noalloc": [_p] * 8 + [_i64] * 6 + [_i32, _i32, _f, _i32, _p, _i64, _p],
@@ -43,7 +48,7 @@ SIGNATURES = {
     "macai_gdr_probe_mfma_flops": [_i32, _i32, _i32],
 }
 # the rest return an int status
-RESTYPES = {"macai_gdr_conv_partials": _i64, "macai_gdr_forward_workspace": _i64, "macai_gdr_probe_mfma_flops": _i64}
+RESTYPES = {"macai_gdr_conv_partials": _i64, "macai_gdr_gates_partials": _i64, "macai_gdr_forward_workspace": _i64, "macai_gdr_probe_mfma_flops": _i64}
 
 _lib = None
 _fns = {}        # name -> the library's function object (a lookup per call costs host time on every launch)

@@ -97,13 +97,21 @@ class ConvQKV(torch.autograd.Function):
             raise RuntimeError("macai's convolution path runs on a HIP device (MI355X); got " + str(x.device))
         sp = _Split(x.shape, kd, dk, rep, dv, repeat)
         src = _dense(x)
-        taps = weight.detach().reshape(sp.C, TAPS).to(torch.float32).contiguous()
+        # the taps as the kernels read them, and their float32 copy for the backward: the kernel writes it for 2-byte
+        # weights, a float32 weight is its own
+        w = weight.detach().reshape(sp.C, TAPS)
+        if w.dtype in DTYPES[1:] and src.numel():
+            w = _dense(w)
+        else:
+            w = w.to(torch.float32).contiguous()
+        taps = w if w.dtype == torch.float32 else torch.empty(sp.C, TAPS, dtype=torch.float32, device=x.device)
         q = torch.empty(sp.qk_shape, dtype=x.dtype, device=x.device)
         k = torch.empty_like(q)
         v = torch.empty(sp.v_shape, dtype=v_dtype, device=x.device)
         if src.numel():
             with _on(x.device):
-                N.call("macai_gdr_conv_fwd", N.ptr(src), N.ptr(taps), N.ptr(q), N.ptr(k), N.ptr(v), *sp.dims(),
+                N.call("macai_gdr_conv_fwd_typed", N.ptr(src), N.ptr(w), N.dtype_code(w.dtype, True),
+                       None if taps is w else N.ptr(taps), N.ptr(q), N.ptr(k), N.ptr(v), *sp.dims(),
                        N.dtype_code(x.dtype, True), N.dtype_code(v_dtype, True), N.stream_of(src))
         ctx.save_for_backward(src, taps)
         ctx.split, ctx.v_dtype = sp, v_dtype
@@ -120,17 +128,18 @@ class ConvQKV(torch.autograd.Function):
         gv = _upstream(grad_v, sp.v_shape, ctx.v_dtype, dev)
         dx = torch.empty_like(src)
         train_w = ctx.needs_input_grad[1]
+        w_shape, w_dtype = ctx.w_meta
+        dw_dtype = w_dtype if w_dtype in DTYPES else torch.float32     # the kernel writes dw in the weight's type
         partials = dw = None
         if train_w:
             partials = torch.empty(N.lib().macai_gdr_conv_partials(sp.B, sp.T, sp.C), dtype=torch.float32, device=dev)
-            dw = torch.zeros(sp.C, TAPS, dtype=torch.float32, device=dev)
+            dw = (torch.empty if src.numel() else torch.zeros)(w_shape, dtype=dw_dtype, device=dev)
         if src.numel():
             with _on(dev):
-                N.call("macai_gdr_conv_bwd", N.ptr(src), N.ptr(taps), N.ptr(gq), N.ptr(gk), N.ptr(gv), N.ptr(dx),
-                       N.ptr(partials), N.ptr(dw), *sp.dims(), N.dtype_code(src.dtype, True),
-                       N.dtype_code(ctx.v_dtype, True), N.stream_of(src))
-        w_shape, w_dtype = ctx.w_meta
-        grad_w = dw.view(w_shape).to(w_dtype) if train_w else None
+                N.call("macai_gdr_conv_bwd_typed", N.ptr(src), N.ptr(taps), N.ptr(gq), N.ptr(gk), N.ptr(gv), N.ptr(dx),
+                       N.ptr(partials), N.ptr(dw), N.dtype_code(dw_dtype, True), *sp.dims(),
+                       N.dtype_code(src.dtype, True), N.dtype_code(ctx.v_dtype, True), N.stream_of(src))
+        grad_w = dw.to(w_dtype) if train_w else None
         return (dx if ctx.needs_input_grad[0] else None), grad_w, None, None, None, None, None, None
 
 

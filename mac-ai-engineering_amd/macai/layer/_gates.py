@@ -70,13 +70,22 @@ class Gates(torch.autograd.Function):
             raise RuntimeError("macai's gates run on a HIP device (MI355X); got " + str(b.device))
         heads = A_log.shape[0]
         pre_b, pre_a = _dense(b), _dense(a)
-        rate_log, bias = _f32(A_log), _f32(dt_bias)
+        f32 = torch.float32
+        if pre_b.numel() and not (A_log.dtype == dt_bias.dtype == f32):
+            # 2-byte parameters: the kernel reads them as they are and writes the float32 copies the backward takes
+            params = torch.empty(2, heads, dtype=f32, device=b.device)
+            p_rate, p_bias = A_log.detach().contiguous(), dt_bias.detach().contiguous()
+            rate_log, bias = params[0], params[1]
+        else:
+            params = None
+            rate_log, bias = p_rate, p_bias = _f32(A_log), _f32(dt_bias)
         beta = torch.empty(pre_b.shape, dtype=torch.float32, device=b.device)
         g = torch.empty_like(beta)
         if pre_b.numel():
             with _on(b.device):
-                N.call("macai_gdr_gates_fwd", N.ptr(pre_b), N.ptr(pre_a), N.ptr(rate_log), N.ptr(bias), N.ptr(beta),
-                       N.ptr(g), pre_b.numel(), heads, N.dtype_code(b.dtype, True), N.stream_of(pre_b))
+                N.call("macai_gdr_gates_fwd_typed", N.ptr(pre_b), N.ptr(pre_a), N.ptr(p_rate),
+                       N.dtype_code(p_rate.dtype, True), N.ptr(p_bias), N.dtype_code(p_bias.dtype, True), N.ptr(params),
+                       N.ptr(beta), N.ptr(g), pre_b.numel(), heads, N.dtype_code(b.dtype, True), N.stream_of(pre_b))
         ctx.save_for_backward(pre_b, pre_a, rate_log, bias)
         ctx.param_dtypes = (A_log.dtype, dt_bias.dtype)
         return beta, g
@@ -89,17 +98,25 @@ class Gates(torch.autograd.Function):
         gg = torch.zeros(pre_b.shape, dtype=torch.float32, device=dev) if grad_g is None else _f32(grad_g)
         d_b, d_a = torch.empty_like(pre_b), torch.empty_like(pre_a)
         need_rate, need_bias = ctx.needs_input_grad[2], ctx.needs_input_grad[3]
+        rate_dt, bias_dt = ctx.param_dtypes
+        n = pre_b.numel()
         d_rate = d_bias = None
         if need_rate or need_bias:
-            d_rate = torch.zeros(heads, dtype=torch.float32, device=dev)
-            d_bias = torch.zeros(heads, dtype=torch.float32, device=dev)
-        if pre_b.numel():
+            new = torch.empty if n else torch.zeros
+            d_rate, d_bias = (new(heads, dtype=dt, device=dev) for dt in (rate_dt, bias_dt))
+        if n:
+            code, stream = N.dtype_code(pre_b.dtype, True), N.stream_of(pre_b)
             with _on(dev):
-                N.call("macai_gdr_gates_bwd", N.ptr(pre_b), N.ptr(pre_a), N.ptr(rate_log), N.ptr(bias), N.ptr(gb),
-                       N.ptr(gg), N.ptr(d_b), N.ptr(d_a), N.ptr(d_rate), N.ptr(d_bias), pre_b.numel(), heads,
-                       N.dtype_code(pre_b.dtype, True), N.stream_of(pre_b))
-        rate_dt, bias_dt = ctx.param_dtypes
-        return (d_b, d_a, d_rate.to(rate_dt) if need_rate else None, d_bias.to(bias_dt) if need_bias else None)
+                if d_rate is None:
+                    N.call("macai_gdr_gates_bwd", N.ptr(pre_b), N.ptr(pre_a), N.ptr(rate_log), N.ptr(bias), N.ptr(gb),
+                           N.ptr(gg), N.ptr(d_b), N.ptr(d_a), None, None, n, heads, code, stream)
+                else:
+                    part = torch.empty(N.lib().macai_gdr_gates_partials(n, heads), dtype=torch.float64, device=dev)
+                    N.call("macai_gdr_gates_bwd_typed", N.ptr(pre_b), N.ptr(pre_a), N.ptr(rate_log), N.ptr(bias),
+                           N.ptr(gb), N.ptr(gg), N.ptr(d_b), N.ptr(d_a), N.ptr(part), N.ptr(d_rate),
+                           N.dtype_code(rate_dt, True), N.ptr(d_bias), N.dtype_code(bias_dt, True), n, heads, code,
+                           stream)
+        return d_b, d_a, (d_rate if need_rate else None), (d_bias if need_bias else None)
 
 
 def gates(b: torch.Tensor, a: torch.Tensor, A_log: torch.Tensor, dt_bias: torch.Tensor):

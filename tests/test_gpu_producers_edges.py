@@ -1,0 +1,57 @@
+"""The producers' kernels at the edges of their tiles, against the float64 oracle: the convolution's blocks of 8 and 16
+time steps and tiles of 64, channel counts that leave lanes of a wave past the channels, parameters in every type (read
+and written in it by the kernels), and the gates' backward with heads that do not divide a workgroup's 256 lanes, more
+heads than that, and one or several rows a lane.  Bounds: a result rounded once to a type of p significant bits is off
+by at most 2^-p of itself, and float32 sums and exponentials before it by a few 2^-24 of their terms; the bar is 2^-p
+plus 2^-20 of the 2-norm (eight such roundings of terms that cancel by half)."""
+import pytest
+import torch
+
+from macai.layer import conv_qkv, gates
+from oracle import producers as P
+from oracle.gdr import rel
+
+pytestmark = pytest.mark.gpu
+F64 = torch.float64
+BITS = {torch.float32: 24, torch.bfloat16: 8, torch.float16: 11}
+
+
+def _draw(shape, dtype, gen, scale=1.0):
+    return (torch.randn(shape, generator=gen, dtype=F64) * scale).to(dtype)
+
+
+def _compare(fused, ref, xs, gen):
+    leaves = [x.cuda().requires_grad_(True) for x in xs]
+    exact = [x.to(F64).requires_grad_(True) for x in xs]
+    outs, refs = fused(*leaves), ref(*exact)
+    ups = [_draw(o.shape, o.dtype, gen) for o in outs]
+    got = list(outs) + list(torch.autograd.grad(outs, leaves, [u.cuda() for u in ups]))
+    want = list(refs) + list(torch.autograd.grad(refs, exact, [u.to(F64) for u in ups]))
+    for i, (x, y) in enumerate(zip(got, want)):
+        e = rel(x.detach().cpu().double(), y.detach())
+        assert e < 2.0 ** -BITS[x.dtype] + 2.0 ** -20, (i, x.dtype, e)
+
+
+@pytest.mark.parametrize("dtype,wdtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                          (torch.float16, torch.bfloat16), (torch.float32, torch.float16)])
+@pytest.mark.parametrize("T", [1, 3, 8, 16, 17, 61, 64, 65, 130])
+def test_conv_blocks_and_channels(T, dtype, wdtype):
+    print("case conv edges", T, dtype, wdtype, flush=True)
+    gen = torch.Generator().manual_seed(T)
+    for kd, dk, rep, dv, repeat in ((8, 8, 1, 8, False), (72, 24, 2, 16, True), (256, 64, 1, 64, False)):
+        C = 2 * kd + kd // dk * rep * dv
+        x, w = _draw((2, T, C), dtype, gen), _draw((C, 1, 4), wdtype, gen, 0.3)
+        _compare(lambda a, b: conv_qkv(a, b, kd, dk, rep, dv, repeat, dtype),
+                 lambda a, b: P.conv_qkv(a, b, kd, dk, rep, dv, repeat), [x, w], gen)
+
+
+@pytest.mark.parametrize("dtype,ptypes", [(torch.bfloat16, (torch.bfloat16, torch.bfloat16)),
+                                          (torch.float32, (torch.float32, torch.float32)),
+                                          (torch.bfloat16, (torch.float32, torch.float16))])
+@pytest.mark.parametrize("rows,H", [(1, 1), (5, 3), (700, 48), (3, 256), (2, 257), (600, 300), (9000, 16)])
+def test_gates_rows_and_heads(rows, H, dtype, ptypes):
+    print("case gates edges", rows, H, dtype, ptypes, flush=True)
+    gen = torch.Generator().manual_seed(rows + H)
+    xs = [_draw((rows, H), dtype, gen), _draw((rows, H), dtype, gen, 3.0), _draw((H,), ptypes[0], gen),
+          _draw((H,), ptypes[1], gen)]
+    _compare(gates, P.gates, xs, gen)
