@@ -801,6 +801,9 @@ struct StateFwdLds {
   // (whole 32-row fragments in each half), both halves' slots and a stage in LDS, and at most 5 waves (two column
   // slices): at 9 waves a wave has 168 registers and the pass spills
   static constexpr bool KS_OK = KS == 2 && sizeof(MT) == 4 && (DK == 64 || DK == 128) && !DIRECT && NW <= 2;
+  // one stage only (the output pass at DK = 128: 119 KB a chunk): its tiles are refilled one by one, each as soon as the
+  // chunk's products are done with it, instead of all of them between two chunks
+  static constexpr bool PHASED = KS_OK && OUT && NBUF == 1;
 };
 
 // The key-split float32 pass (the compute waves of state_fwd_body with KS = 2).  The 16x16x4 float32 MFMA takes a
@@ -811,6 +814,10 @@ struct StateFwdLds {
 // each forms the output's row blocks 2 h, 2 h + 1 from the whole S (the partner's half from LDS) and Vn.  Per wave
 // that is 208-224 MFMAs a chunk at DK = 128 against 432 for one wave.  The single-wave form sums the two halves of
 // W S the same way, so both give the same bits.
+// Where the chunk's tiles fit LDS once only (PHASED), W is refilled behind the second and third group of products (S's
+// update, the output), K behind the output and the next W S, Q and M behind W S and the update, a barrier after each
+// group: the loader used to copy all 119 KB between two chunks, which took as long as the products.  At 32 head-rows of
+// 16 chunks 118 -> 84 us (of that the float32 MFMAs are 48: 224 of 32 cycles a wave and chunk).
 template <int DK, int NW, bool OUT, bool STORE>
 __device__ __forceinline__ void state_fwd_ks(const StateFwdArgs& a, float* lds, int hr, int slice, int cb, int ce,
                                              size_t crow, int tb) {
@@ -820,6 +827,7 @@ __device__ __forceinline__ void state_fwd_ks(const StateFwdArgs& a, float* lds, 
   using GM = typename L::GM;
   constexpr int ND = DK / 16, NH = ND / 2, PH = NH / 2;   // state tiles; a wave's tiles and its 32-row k-blocks
   constexpr int O_KE = L::O_KE, O_Q = L::O_Q, O_M = L::O_M, SZ = L::SZ, NBUF = L::NBUF;
+  constexpr bool PHASED = L::PHASED;
   const int T = a.T, H = a.H, DV = a.DV, NT = a.NT;
   const int h = hr % H;
   const int l = lane_id(), w = wave_id(), j = l >> 4;
@@ -845,7 +853,7 @@ __device__ __forceinline__ void state_fwd_ks(const StateFwdArgs& a, float* lds, 
   if (cb < ce) {
     loadU(cb, Un);
     gln = a.GL[crow * NT + cb];
-    if (NBUF == 2) lds_barrier();        // the first chunk is in LDS
+    if (NBUF == 2 || PHASED) lds_barrier();   // the first chunk (PHASED: its W) is in LDS
   }
   for (int c = cb; c < ce; ++c) {
     const size_t bhc = crow * NT + c;
@@ -865,7 +873,7 @@ __device__ __forceinline__ void state_fwd_ks(const StateFwdArgs& a, float* lds, 
 #pragma unroll
         for (int r = 0; r < 4; ++r) Scc[(16 * di + r) * DV] = S[di][r];
     }
-    if (NBUF == 1) lds_barrier();        // chunk c is in LDS
+    if (NBUF == 1 && !PHASED) lds_barrier();   // chunk c is in LDS
     const MT* st = lds + buf * SZ;
     const MT* tW = st;
     const MT* tK = st + O_KE;
@@ -889,7 +897,7 @@ __device__ __forceinline__ void state_fwd_ks(const StateFwdArgs& a, float* lds, 
       for (int mi = 0; mi < 4; ++mi) mma(P[mi], frag_tile<MT, GW>(tW, 16 * mi, 32 * (kh * PH + p)), Sf[p]);
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) *reinterpret_cast<f4*>(xme + L::XS + (mi * 64 + l) * 4) = P[mi];
-    lds_barrier();                         // the pair's halves are in LDS
+    lds_barrier();                         // the pair's halves are in LDS (PHASED: K too, and W is free)
     f4 Vn[4];
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) Vn[mi] = U[mi] - (P[mi] + *reinterpret_cast<const f4*>(xpa + L::XS + (mi * 64 + l) * 4));
@@ -910,6 +918,7 @@ __device__ __forceinline__ void state_fwd_ks(const StateFwdArgs& a, float* lds, 
 #pragma unroll
       for (int p = 0; p < 2; ++p) mma(S[di], frag_tile_tr<MT, GW>(tK, 32 * p, r0 + 16 * di), Vf[p]);
     }
+    if constexpr (PHASED) lds_barrier();   // Q and M are in LDS, K is free
     if constexpr (OUT) {
       // rows 16 mi of O^T = S^T (diag(gamma) Q)^T + Vn^T M^T for mi = 2 kh, 2 kh + 1, from the whole S (fragments of
       // rows 0 .. DK / 2 - 1 in S0, the rest in S1)
@@ -1011,6 +1020,36 @@ __device__ __forceinline__ void state_fwd_body(const StateFwdArgs& a, MT* lds, i
         GM::template dma_planned<1>(st + O_M, (const MT*)a.M + bhc * C * C, offM, 0);
       }
     };
+    if constexpr (L::PHASED) {             // see state_fwd_ks; copies land in issue order
+      constexpr int NG = GW::NI, NM = GM::NI;
+      auto tile = [&](int o, const void* g, int c) {
+        GW::template dma_planned<1>(lds + o, (const MT*)g + (crow * NT + c) * C * DK, offW, 0);
+      };
+      if (cb >= ce) return;
+      tile(0, a.W, cb);
+      tile(O_KE, a.Ke, cb);
+      wait_vmcnt<NG>();
+      lds_barrier();                       // the first W is in
+      for (int c = cb; c < ce; ++c) {
+        tile(O_Q, a.Qg, c);
+        GM::template dma_planned<1>(lds + O_M, (const MT*)a.M + (crow * NT + c) * C * C, offM, 0);
+        wait_vmcnt<NG + NM>();             // K is in
+        lds_barrier();
+        if (c + 1 < ce) {
+          tile(0, a.W, c + 1);
+          wait_vmcnt<NG>();                // Q and M are in
+        } else {
+          wait_dma();
+        }
+        lds_barrier();
+        if (c + 1 < ce) {
+          tile(O_KE, a.Ke, c + 1);
+          wait_vmcnt<NG>();                // the next W is in
+        }
+        lds_barrier();
+      }
+      return;
+    }
     if (NBUF == 2) {
       if (cb < ce) {
         issue(cb, 0);
@@ -1630,14 +1669,18 @@ struct StateBwdLds {
       DIRECT ? 0 : Buffers<SZ * (int)sizeof(MT), (STG + SCAL + EX) * (int)sizeof(MT) + TOUCH_SINK>::N;
   static constexpr int O_STG = NBUF * SZ, O_SCAL = O_STG + STG, O_EX = O_SCAL + SCAL;
   static constexpr int ELEMS = O_EX + EX;
-  // see StateFwdLds::KS_OK
+  // see StateFwdLds::KS_OK and PHASED
   static constexpr bool KS_OK = KS == 2 && sizeof(MT) == 4 && (DK == 64 || DK == 128) && !DIRECT && NW <= 2;
+  static constexpr bool PHASED = KS_OK && NBUF == 1;
 };
 
 // The key-split float32 reverse pass (the compute waves of state_bwd_body with KS = 2; see state_fwd_ks): wave
 // 2 s + h holds rows [h DK / 2, (h + 1) DK / 2) of its slice's dS.  Per chunk each forms its half of diag(e) K^ dS
 // (with M^T dO for row blocks 2 h, 2 h + 1), the pair exchanges the halves through LDS and both take dVn as their sum,
 // then each updates its own rows of dS.  Per wave 208-224 MFMAs a chunk at DK = 128 against 432 for one wave.
+// Where the chunk's tiles fit LDS once only (PHASED, DK = 128), the first half's tiles (K, M, dO) are refilled behind
+// the second half (Q^T dO, W^T dVn) and the second's (Q, W) behind the next chunk's first: 128 -> 90 us at 32
+// head-rows of 16 chunks.
 template <int DK, int NW>
 __device__ __forceinline__ void state_bwd_ks(const StateBwdArgs& a, float* lds, int hr, int slice, int cb, int ce,
                                              size_t crow, int tb) {
@@ -1660,7 +1703,7 @@ __device__ __forceinline__ void state_bwd_ks(const StateBwdArgs& a, float* lds, 
 
   f4 dS[NH];
   load_state(dS, a.dsT, (size_t)hr * DK * DV + (size_t)r0 * DV, DV, col);
-  if (cb < ce && NBUF == 2) lds_barrier();   // the last chunk is in LDS
+  if (cb < ce && (NBUF == 2 || L::PHASED)) lds_barrier();   // the last chunk (PHASED: its K, M, dO) is in LDS
   for (int c = ce - 1, it = 0; c >= cb; --c, ++it) {
     const int buf = (NBUF == 2) ? (it & 1) : 0;
     const size_t bhc = crow * NT + c;
@@ -1675,7 +1718,7 @@ __device__ __forceinline__ void state_bwd_ks(const StateBwdArgs& a, float* lds, 
 #pragma unroll
         for (int r = 0; r < 4; ++r) dSc[(16 * di + r) * dv] = dS[di][r];
     }
-    if (NBUF == 1) lds_barrier();        // chunk c is in LDS
+    if (NBUF == 1 && !L::PHASED) lds_barrier();   // chunk c is in LDS
     const int* sc = (const int*)(lds + L::O_SCAL) + 4 * buf;
     const float gl = __int_as_float(sc[0]);
     const int t0 = sc[1], tend = sc[2];
@@ -1710,7 +1753,7 @@ __device__ __forceinline__ void state_bwd_ks(const StateBwdArgs& a, float* lds, 
       P[mi] = acc;
       *reinterpret_cast<f4*>(xme + (mi * 64 + l) * 4) = acc;
     }
-    lds_barrier();                         // the pair's halves are in LDS
+    lds_barrier();                         // the pair's halves are in LDS (PHASED: Q, W too; K, M, dO are free)
     f4 dV[4];
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) dV[mi] = P[mi] + *reinterpret_cast<const f4*>(xpa + (mi * 64 + l) * 4);
@@ -1778,7 +1821,13 @@ __device__ __forceinline__ void state_bwd_body(const StateBwdArgs& a, MT* lds, i
     GK::template plan<1>(offK, 0, DK);
     GM::template plan<1>(offM, 0, C);
     GO::template plan<1>(offO, 0, (int)o_pitch);
-    auto issue = [&](int c, int buf) {
+    auto issue2 = [&](int c, int buf) {    // the tiles of the second half
+      MT* st = lds + buf * SZ;
+      const size_t bhc = crow * NT + c;
+      GK::dma(st + O_Q, (const MT*)a.Qg + bhc * C * DK, DK, 0, 1);
+      GK::dma(st + O_W, (const MT*)a.W + bhc * C * DK, DK, 0, 1);
+    };
+    auto issue = [&](int c, int buf) {     // the chunk's tiles (PHASED: those of the first half)
       MT* st = lds + buf * SZ;
       const size_t bhc = crow * NT + c;
       int t0, tend;
@@ -1786,8 +1835,7 @@ __device__ __forceinline__ void state_bwd_body(const StateBwdArgs& a, MT* lds, i
       const MT* og = (const MT*)a.dO + o_base + (size_t)t0 * o_pitch + vg;
       if constexpr (KS == 2) {             // addresses formed per copy: the planned offsets (59 registers at DK = 128)
         GK::dma(st, (const MT*)a.Ke + bhc * C * DK, DK, 0, 1);   // spill at 5 waves' 256 registers a wave
-        GK::dma(st + O_Q, (const MT*)a.Qg + bhc * C * DK, DK, 0, 1);
-        GK::dma(st + O_W, (const MT*)a.W + bhc * C * DK, DK, 0, 1);
+        if constexpr (!L::PHASED) issue2(c, buf);
         GM::dma(st + O_M, (const MT*)a.M + bhc * C * C, C, 0, 1);
         GO::dma(st + O_O, og, o_pitch, 0, 1, tend - t0);
       } else {
@@ -1820,6 +1868,21 @@ __device__ __forceinline__ void state_bwd_body(const StateBwdArgs& a, MT* lds, i
                      o_pitch * sizeof(MT), tend - t0);
       wait_vmcnt<TOUCH_LOADS>();
     };
+    if constexpr (L::PHASED) {             // see state_bwd_ks
+      if (cb >= ce) return;
+      issue(ce - 1, 0);
+      wait_dma();
+      lds_barrier();
+      for (int c = ce - 1; c >= cb; --c) {
+        issue2(c, 0);
+        wait_dma();
+        lds_barrier();
+        if (c > cb) issue(c - 1, 0);
+        wait_dma();
+        lds_barrier();
+      }
+      return;
+    }
     if (NBUF == 2) {
       if (cb < ce) {
         issue(ce - 1, 0);
