@@ -2058,7 +2058,8 @@ __device__ __forceinline__ Frag<MT> zero_frag() {
 }
 
 // The fp32 per-chunk backward (bf16 operands take chunk_bwd8_kernel): one workgroup of NW = cb32_waves(DK) waves per
-// (chunk, head, batch row), fragments read straight from global memory (fp32 tiles do not fit LDS).  The prologue's
+// (chunk, head, batch row), q, k, v, A and the states' fragments read straight from global memory (LDS holds the other
+// three fp32 tiles at most: TILED).  The prologue's
 // row scales (q^ = q rq DK^-1/2, k^ = k rk) are applied to the products' rows and columns, and folded into the stored
 // dM and Z, so the raw inputs are the MFMA operands.  Wave w owns key-column blocks w, w + NW, ... of the [C x DK]
 // products and value-column blocks w, w + NW, ..., and of the [C x C] ones column block w % 4, row tiles
@@ -2076,11 +2077,22 @@ __global__ void __launch_bounds__(64 * cb32_waves(DK)) chunk_bwd_kernel(ChunkBwd
   constexpr int RH = NW / 4, TPW = 4 / RH;   // row groups of the C x C tiles, row tiles a wave owns there
   constexpr int NBD = DK / 16;            // 16-column blocks of the key width
   constexpr int NBW = (NBD + NW - 1) / NW;   // most blocks a wave owns
+  // TILED: the dO, Vn and dVn tiles in LDS while B and the products of C read them, in the place that C's results then
+  // take.  Every wave reads all three tiles in B and half of them in C, over 1 MB a chunk-head through the vector cache
+  // when they are read from memory, at two waves a SIMD to hide its latency: at 512 chunk-heads of 128 x 128 177 us that
+  // way, 148 from LDS (the float32 MFMAs alone 64).  The widths that need 4 waves or take DV at run time do not fit.
+  constexpr bool TILED = NW == 8 && DVT > 0;
+  using GT = Tile<MT, C, DVT ? DVT : 32>;
+  constexpr int CC = C * CP, TILES = TILED && 3 * GT::ELEMS > 4 * CC ? 3 * GT::ELEMS : 4 * CC;
   __shared__ __attribute__((aligned(16))) MT sdW[C * KP];   // dW = -dVn S_c^T
-  __shared__ __attribute__((aligned(16))) MT sdMk[C * CP];  // dM diag(rk):            [t][s] = dM[t][s] rk_s
-  __shared__ __attribute__((aligned(16))) MT sdMq[C * CP];  // dM^T diag(rq DK^-1/2):  [t][s] = dM[s][t] rq_s qs
-  __shared__ __attribute__((aligned(16))) MT sZk[C * CP];   // Z diag(rk), Z = diag(beta) P + (diag(beta) P)^T
-  __shared__ __attribute__((aligned(16))) MT sdA[C * CP];   // dA
+  __shared__ __attribute__((aligned(16))) MT tiles[TILES];
+  MT* const sdMk = tiles;                                   // dM diag(rk):            [t][s] = dM[t][s] rk_s
+  MT* const sdMq = tiles + CC;                              // dM^T diag(rq DK^-1/2):  [t][s] = dM[s][t] rq_s qs
+  MT* const sZk = tiles + 2 * CC;                           // Z diag(rk), Z = diag(beta) P + (diag(beta) P)^T
+  MT* const sdA = tiles + 3 * CC;                           // dA
+  MT* const tO = tiles;
+  MT* const tVn = tiles + GT::ELEMS;
+  MT* const tdVn = tiles + 2 * GT::ELEMS;
   __shared__ ChunkScalars cs;
   __shared__ float rk[C], rq[C];
   __shared__ float part[NPART][NW][C];
@@ -2109,6 +2121,11 @@ __global__ void __launch_bounds__(64 * cb32_waves(DK)) chunk_bwd_kernel(ChunkBwd
   const MT* Ac = (const MT*)a.A + bhc * C * C;
   const float qs = a.q_scale;
 
+  if constexpr (TILED) {
+    GT::dma(tO, dO + (size_t)t0 * v_pitch, v_pitch, w, NW, nrows);
+    GT::dma(tVn, Vnc, DV, w, NW);
+    GT::dma(tdVn, dVc, DV, w, NW);
+  }
   if (w == 0) chunk_scalars(cs, a.g, a.beta, s_base, H, t0, T);
   if (a.l2norm) {
     if constexpr (NW == 8) {               // k's norms on waves 0-3, q's on 4-7 (the same sums as on one wave set)
@@ -2122,7 +2139,13 @@ __global__ void __launch_bounds__(64 * cb32_waves(DK)) chunk_bwd_kernel(ChunkBwd
     rk[threadIdx.x] = (int)threadIdx.x < nrows ? 1.f : 0.f;
     rq[threadIdx.x] = (int)threadIdx.x < nrows ? 1.f : 0.f;
   }
+  if constexpr (TILED) wait_dma();
   __syncthreads();
+  if (TILED && nrows < C) {                // dO rows past the end: zeros
+    for (int i = threadIdx.x; i < (C - nrows) * (DV / 4); i += blockDim.x)
+      *reinterpret_cast<f4*>(tO + (nrows + i / (DV / 4)) * GT::PITCH + 4 * (i % (DV / 4))) = f4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+  }
 
   // operand accessors: raw rows (zero past the sequence end)
   auto fq = [&](int row0, int k0) { return frag_k_seq<MT, IT>(q, qk_pitch, t0, T, row0, k0, One()); };
@@ -2137,9 +2160,18 @@ __global__ void __launch_bounds__(64 * cb32_waves(DK)) chunk_bwd_kernel(ChunkBwd
     if constexpr (EAGER) return frag_rows_eager<MT, IT>(k, qk_pitch, t0, T, krow0, col, One());
     else return frag_rows<MT, IT>(k, qk_pitch, t0, T, krow0, col, One());
   };
-  auto fO = [&](int row0, int k0) { return frag_k_seq<MT, MT>(dO, v_pitch, t0, T, row0, k0, One()); };
-  auto fVn = [&](int row0, int k0) { return frag_k<MT, MT>(Vnc, DV, row0, k0); };
-  auto fdVn = [&](int row0, int k0) { return frag_k<MT, MT>(dVc, DV, row0, k0); };
+  auto fO = [&](int row0, int k0) {
+    if constexpr (TILED) return frag_tile<MT, GT>(tO, row0, k0);
+    else return frag_k_seq<MT, MT>(dO, v_pitch, t0, T, row0, k0, One());
+  };
+  auto fVn = [&](int row0, int k0) {
+    if constexpr (TILED) return frag_tile<MT, GT>(tVn, row0, k0);
+    else return frag_k<MT, MT>(Vnc, DV, row0, k0);
+  };
+  auto fdVn = [&](int row0, int k0) {
+    if constexpr (TILED) return frag_tile<MT, GT>(tdVn, row0, k0);
+    else return frag_k<MT, MT>(dVc, DV, row0, k0);
+  };
   auto fdVnrows = [&](int krow0, int col) {
     if constexpr (EAGER) return frag_rows_eager<MT, MT>(dVc, DV, 0, C, krow0, col, One());
     else return frag_rows<MT, MT>(dVc, DV, 0, C, krow0, col, One());
@@ -2297,6 +2329,7 @@ __global__ void __launch_bounds__(64 * cb32_waves(DK)) chunk_bwd_kernel(ChunkBwd
       mma(Tb[i], fd[i], bv);
     }
   }
+  if constexpr (TILED) __syncthreads();    // the tiles are read: C's results take their place
   float gm[TPW][4], KG[TPW][4];
   {
     float cR1 = 0.f;
