@@ -1265,8 +1265,14 @@ __device__ __forceinline__ void state_fwd_body(const StateFwdArgs& a, MT* lds, i
   }
 }
 
+// The launch bound the forward passes are compiled for.  LDS holds them to one workgroup a CU, and at four waves or fewer
+// the compiler counts one wave a SIMD and takes the MFMAs' accumulators in AGPRs, which no VALU instruction reads (96
+// moves a chunk in the two-wave float32 output pass).  Compiled for five waves that pass has 256 registers, enough, and
+// no moves: 84 -> 82 us at 32 head-rows of 16 chunks, the store pass 54 -> 52.  (The reverse pass spills at 256.)
+constexpr int fwd_threads(int ks, int nw) { return ks == 2 && nw == 1 ? 320 : 64 * (ks * nw + 1); }
+
 template <typename MT, int DK, int NW, bool OUT, bool STORE, bool MAP = false, int KS = 1>
-__global__ void __launch_bounds__(64 * (KS * NW + 1)) state_fwd_kernel(StateFwdArgs a) {
+__global__ void __launch_bounds__(fwd_threads(KS, NW)) state_fwd_kernel(StateFwdArgs a) {
   __shared__ __attribute__((aligned(1024))) MT lds[StateFwdLds<MT, DK, OUT, STORE, NW, KS>::ELEMS];
   state_fwd_body<MT, DK, NW, OUT, STORE, MAP, KS>(a, lds, blockIdx.x);
 }
