@@ -51,7 +51,7 @@
 extern "C" {
 #endif
 
-#define MACAI_GDR_ABI_VERSION 14
+#define MACAI_GDR_ABI_VERSION 15
 
 /* dtype codes (the rule takes F32 and BF16; the producers also F16) */
 #define MACAI_GDR_F32 0
@@ -140,6 +140,18 @@ int macai_gdr_chunk_bwd(const void* q, const void* k, const void* v, const float
                         const void* dVn, void* dq, void* dk, void* dv, float* dg, float* dbeta, int64_t B, int64_t T,
                         int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype, int32_t use_l2norm,
                         float q_scale, const int32_t* pack, int64_t NT, void* stream);
+
+/* The same with the gradients of a key head's value heads summed in the kernel: dq, dk [B, T, Hk, DK], the bits of
+ * macai_gdr_chunk_bwd followed by macai_gdr_group_sum on each, without their per-head arrays and launches.  Taken where
+ * macai_gdr_chunk_bwd_folds returns 1 for the shape on the current device (bf16, two value heads a key head, DK = DV and
+ * more chunk-heads than the device runs at once, in whole pairs); EUNSUP elsewhere. */
+int macai_gdr_chunk_bwd_folds(int64_t B, int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype,
+                              const int32_t* pack, int64_t NT);
+int macai_gdr_chunk_bwd_folded(const void* q, const void* k, const void* v, const float* g, const float* beta,
+                               const void* dO, const void* A, const float* Sc, const float* dSn, const void* Vn,
+                               const void* dVn, void* dq, void* dk, void* dv, float* dg, float* dbeta, int64_t B,
+                               int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype,
+                               int32_t use_l2norm, float q_scale, const int32_t* pack, int64_t NT, void* stream);
 
 /* The inference forward in one call: macai_gdr_prep (without A) then macai_gdr_state_fwd with the output (flags 0),
  * the per-chunk operands W, U, Ke, GL, Qg, M carved from `workspace` (256-byte aligned, at least

@@ -8,15 +8,18 @@
 
 namespace gdr {
 
-void cb8_launch(const ChunkBwdArgs& a, int DK, int DV, bool xn, int wgs, int units, dim3 grid, hipStream_t st) {
+void cb8_launch(const ChunkBwdArgs& a, int DK, int DV, bool xn, bool fold, int wgs, int units, dim3 grid,
+                hipStream_t st) {
 #define CB8_DISPATCH_DK(...)                                   \
   switch (DK) {                                                \
     case 32: { constexpr int DKC = 32; __VA_ARGS__; } break;   \
     case 64: { constexpr int DKC = 64; __VA_ARGS__; } break;   \
     default: { constexpr int DKC = 128; __VA_ARGS__; } break;  \
   }
-  if (xn) {
-    CB8_DISPATCH_DK(hipLaunchKernelGGL((chunk_bwd8xn_kernel<DKC>), dim3((unsigned)wgs), dim3(512), 0, st, a, units));
+  if (fold) {
+    CB8_DISPATCH_DK(hipLaunchKernelGGL((chunk_bwd8xn_kernel<DKC, true>), dim3((unsigned)wgs), dim3(512), 0, st, a, units));
+  } else if (xn) {
+    CB8_DISPATCH_DK(hipLaunchKernelGGL((chunk_bwd8xn_kernel<DKC, false>), dim3((unsigned)wgs), dim3(512), 0, st, a, units));
   } else {
     CB8_DISPATCH_DK(switch (DV) {
       case 32: hipLaunchKernelGGL((chunk_bwd8_kernel<DKC, 32>), grid, dim3(512), 0, st, a); break;

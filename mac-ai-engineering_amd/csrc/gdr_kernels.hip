@@ -2661,7 +2661,11 @@ __device__ __forceinline__ void cb8_stagger(int stagger, unsigned flat) {
 // products) a value block at a time in T1, dL and D, its Vn into tO and its dVn, g and beta in G.  The copies into
 // LDS are issued unseen by the compiler (dma_exact_opaque), so the arrays may be chosen at run time, and each is
 // waited for explicitly.
-template <int DK, int DV>
+// FOLD (two value heads a key head): dq and dk are the key head's [B,T,Hk,DK]; the pair's first value head writes its
+// rows rounded to bf16 there, the second, run by the same workgroup next, adds its own rounded rows to them in float32
+// and rounds once (what macai_gdr_group_sum makes of the two, the same bits): each lane reads back the 16 bytes it wrote
+// itself.
+template <int DK, int DV, bool FOLD = false>
 __device__ __forceinline__ void chunk_bwd8_body(const ChunkBwdArgs& a, const Cb8Lds& L, int unit, int next, bool first,
                                                 bf16* const tO, bf16* const tVn, bf16* const sdW,
                                                 Frag<float> (&s32)[DV / 32], Frag<float> (&sD)[DV / 32], float& gv,
@@ -2701,7 +2705,8 @@ __device__ __forceinline__ void chunk_bwd8_body(const ChunkBwdArgs& a, const Cb8
   asm volatile("" : "+s"(w));
   const int j = l >> 4, n = l & 15, tid = 64 * w + l;
   const size_t qk_base = ((size_t)b * a.T * a.Hk + h / (H / a.Hk)) * DK, qk_pitch = (size_t)a.Hk * DK;
-  const size_t dqk_base = ((size_t)b * a.T * H + h) * DK, dqk_pitch = (size_t)H * DK;   // dq, dk: value heads
+  const size_t dqk_base = FOLD ? qk_base : ((size_t)b * a.T * H + h) * DK;   // dq, dk: value heads, or folded
+  const size_t dqk_pitch = FOLD ? qk_pitch : (size_t)H * DK;
   const size_t v_base = ((size_t)b * a.T * H + h) * DV, v_pitch = (size_t)H * DV;
   const size_t s_base = (size_t)b * a.T * H + h;
   const size_t bhc = ((size_t)b * H + h) * NT + c;
@@ -3267,8 +3272,20 @@ __device__ __forceinline__ void chunk_bwd8_body(const ChunkBwdArgs& a, const Cb8
                    q1 = *reinterpret_cast<const bf16x4*>(tq + row * KP + 8 * u + 4),
                    k0 = *reinterpret_cast<const bf16x4*>(tk + row * KP + 8 * u),
                    k1 = *reinterpret_cast<const bf16x4*>(tk + row * KP + 8 * u + 4);
-      *reinterpret_cast<bf16x8*>(dq + row * dqk_pitch + 8 * u) = bf16x8{q0[0], q0[1], q0[2], q0[3], q1[0], q1[1], q1[2], q1[3]};
-      *reinterpret_cast<bf16x8*>(dk + row * dqk_pitch + 8 * u) = bf16x8{k0[0], k0[1], k0[2], k0[3], k1[0], k1[1], k1[2], k1[3]};
+      bf16x8 xq = {q0[0], q0[1], q0[2], q0[3], q1[0], q1[1], q1[2], q1[3]};
+      bf16x8 xk = {k0[0], k0[1], k0[2], k0[3], k1[0], k1[1], k1[2], k1[3]};
+      bf16x8* const gq8 = reinterpret_cast<bf16x8*>(dq + row * dqk_pitch + 8 * u);
+      bf16x8* const gk8 = reinterpret_cast<bf16x8*>(dk + row * dqk_pitch + 8 * u);
+      if (FOLD && (h & 1)) {
+        const bf16x8 pq = *gq8, pk = *gk8;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          xq[e] = (bf16)((float)pq[e] + (float)xq[e]);
+          xk[e] = (bf16)((float)pk[e] + (float)xk[e]);
+        }
+      }
+      *gq8 = xq;
+      *gk8 = xk;
     }
     for (int i = wt; i < nrows * UV; i += NTH) {
       const int row = i / UV, u = i - row * UV;
@@ -3324,7 +3341,8 @@ __global__ void __launch_bounds__(512) chunk_bwd8_kernel(ChunkBwdArgs a) {
 // each one's reads issued while the one before it computes, so only the first one's load phase is exposed.  The value
 // tiles' arrays rotate: the next unit's dO goes into this one's dW array, its Vn into this one's dO/v array, and its
 // dW array is this one's Vn/dv array.
-template <int D>
+// FOLD: the run goes over chunks of key heads, the two value heads of each in turn (units: chunk-heads).
+template <int D, bool FOLD>
 __global__ void __launch_bounds__(512) chunk_bwd8xn_kernel(ChunkBwdArgs a, int units) {
   CB8_LDS(D, D)
   Frag<float> s32[D / 32], sD[D / 32];
@@ -3332,14 +3350,20 @@ __global__ void __launch_bounds__(512) chunk_bwd8xn_kernel(ChunkBwdArgs a, int u
   bf16 *tO = L.R1, *tVn = L.R2, *sdW = L.R7;
   const int stride = gridDim.x;
   bool first = true;
-  for (int u = blockIdx.x; u < units; u += stride) {
-    const int next = u + stride < units ? u + stride : -1;
-    chunk_bwd8_body<D, D>(a, L, u, next, first, tO, tVn, sdW, s32, sD, gv, bv);
+  // the chunk-head of value head g of key-head chunk u (FOLD), of chunk-head u itself otherwise
+  const int end = FOLD ? units / 2 : units;
+  auto unit_of = [&](int u, int g) { return FOLD ? ((u / a.NT) * 2 + g) * a.NT + u % a.NT : u; };
+  for (int u = blockIdx.x, g = 0; u < end;) {
+    const int nu = FOLD && g == 0 ? u : u + stride, ng = FOLD ? g ^ 1 : 0;
+    const int next = nu < end ? unit_of(nu, ng) : -1;
+    chunk_bwd8_body<D, D, FOLD>(a, L, unit_of(u, g), next, first, tO, tVn, sdW, s32, sD, gv, bv);
     bf16* const t = sdW;
     sdW = tVn;
     tVn = tO;
     tO = t;
     first = false;
+    u = nu;
+    g = ng;
   }
 }
 
@@ -3425,7 +3449,8 @@ __global__ void __launch_bounds__(256) decode_kernel(DecodeArgs a) {
 // this file's device code and is compiled with LLVM's max-memory-clause scheduling strategy (chunk_bwd8 2.5% faster
 // with it; applied to the whole library it slowed state_bwd by 4% and grew the spills of the float32 state kernels).
 // xn: the persistent form (wgs workgroups over `units` chunk-heads); else one chunk-head a workgroup over `grid`.
-void cb8_launch(const ChunkBwdArgs& a, int DK, int DV, bool xn, int wgs, int units, dim3 grid, hipStream_t st);
+void cb8_launch(const ChunkBwdArgs& a, int DK, int DV, bool xn, bool fold, int wgs, int units, dim3 grid,
+                hipStream_t st);
 
 }  // namespace gdr
 
@@ -3821,12 +3846,52 @@ int macai_gdr_state_scan(const float* maps, const float* s0, float* starts, int6
 #endif
 
 #if GDR_IN_PART(5)
+// Whether the per-chunk backward sums the gradients of a key head's value heads itself: bf16 operands on the persistent
+// form (DK = DV, more chunk-heads than CUs) with two value heads a key head, where a workgroup can run both of a key
+// head's in turn without a longer run: 2 ceil(units / 2 / CUs) chunk-heads the longest instead of ceil(units / CUs).
+// (One more chunk-head a run costs about 20 us at 128 x 128.  Folding saves the two group_sum launches and the per-head
+// rows they read: a training step of 1,024 chunk-heads 254 -> 244 us, of 8,192 1,824 -> 1,771.)
+static bool cb8_folds(int64_t units, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int dtype, int64_t cus) {
+  return dtype == MACAI_GDR_BF16 && DK == DV && Hk > 0 && H == 2 * Hk && cus > 0 && units > cus &&
+         units < (int64_t)1 << 30 && 2 * ((units / 2 + cus - 1) / cus) <= (units + cus - 1) / cus;
+}
+
+int macai_gdr_chunk_bwd_folds(int64_t B, int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype,
+                              const int32_t* pack, int64_t NT_packed) {
+  const int64_t chunks = pack ? NT_packed : B * ((T + C - 1) / C);
+  return cb8_folds(chunks * H, H, Hk, DK, DV, dtype, device_cus()) ? 1 : 0;
+}
+
+static int chunk_bwd(const char* what, bool fold, const void* q, const void* k, const void* v, const float* g,
+                     const float* beta, const void* dO, const void* A, const float* Sc, const float* dSn,
+                     const void* Vn, const void* dVn, void* dq, void* dk, void* dv, float* dg, float* dbeta, int64_t B,
+                     int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype, int32_t use_l2norm,
+                     float q_scale, const int32_t* pack, int64_t NT_packed, void* stream);
+
 int macai_gdr_chunk_bwd(const void* q, const void* k, const void* v, const float* g, const float* beta, const void* dO,
                         const void* A, const float* Sc, const float* dSn, const void* Vn,
                         const void* dVn, void* dq, void* dk, void* dv, float* dg, float* dbeta, int64_t B, int64_t T,
                         int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype, int32_t use_l2norm, float q_scale,
                         const int32_t* pack, int64_t NT_packed, void* stream) {
-  const char* what = "macai_gdr_chunk_bwd";
+  return chunk_bwd("macai_gdr_chunk_bwd", false, q, k, v, g, beta, dO, A, Sc, dSn, Vn, dVn, dq, dk, dv, dg, dbeta, B, T,
+                   H, Hk, DK, DV, dtype, use_l2norm, q_scale, pack, NT_packed, stream);
+}
+
+int macai_gdr_chunk_bwd_folded(const void* q, const void* k, const void* v, const float* g, const float* beta,
+                               const void* dO, const void* A, const float* Sc, const float* dSn, const void* Vn,
+                               const void* dVn, void* dq, void* dk, void* dv, float* dg, float* dbeta, int64_t B,
+                               int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype,
+                               int32_t use_l2norm, float q_scale, const int32_t* pack, int64_t NT_packed,
+                               void* stream) {
+  return chunk_bwd("macai_gdr_chunk_bwd_folded", true, q, k, v, g, beta, dO, A, Sc, dSn, Vn, dVn, dq, dk, dv, dg, dbeta,
+                   B, T, H, Hk, DK, DV, dtype, use_l2norm, q_scale, pack, NT_packed, stream);
+}
+
+static int chunk_bwd(const char* what, bool fold, const void* q, const void* k, const void* v, const float* g,
+                     const float* beta, const void* dO, const void* A, const float* Sc, const float* dSn,
+                     const void* Vn, const void* dVn, void* dq, void* dk, void* dv, float* dg, float* dbeta, int64_t B,
+                     int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype, int32_t use_l2norm,
+                     float q_scale, const int32_t* pack, int64_t NT_packed, void* stream) {
   const bool mixed = dtype == MACAI_GDR_BF16_F32;   // bf16 q, k, v and dq, dk, dv; float32 dO and operands
   if (mixed) dtype = MACAI_GDR_F32;
   int64_t NT = 0;
@@ -3852,6 +3917,8 @@ int macai_gdr_chunk_bwd(const void* q, const void* k, const void* v, const float
                  (int)DV, (int)NT, use_l2norm, q_scale, (int)Hk, pack, 0};
   dim3 grid(a.NT, (unsigned)H, pack ? 1u : (unsigned)B);
   const int64_t units = (int64_t)grid.x * grid.y * grid.z;
+  if (fold && !cb8_folds(units, H, Hk, DK, DV, mixed ? MACAI_GDR_BF16_F32 : dtype, device_cus()))
+    return fail(MACAI_GDR_EUNSUP, "%s: this shape takes macai_gdr_chunk_bwd and macai_gdr_group_sum", what);
   bool xn = false;                         // persistent workgroups, one a CU (DK = DV, more chunk-heads than CUs)
   if (dtype != MACAI_GDR_F32) {            // chunk_bwd8 (one workgroup a CU): stagger its first round when more follow
     const int cus = device_cus();
@@ -3881,7 +3948,8 @@ int macai_gdr_chunk_bwd(const void* q, const void* k, const void* v, const float
     LAUNCH_CB(float);
   } else {
     const int cus = xn ? device_cus() : 0;
-    cb8_launch(a, (int)DK, (int)DV, xn, (int)(xn && units > cus ? cus : units), (int)units, grid, st);
+    const int64_t runs = fold ? units / 2 : units;   // folded: a key head's two chunk-heads run in turn
+    cb8_launch(a, (int)DK, (int)DV, xn, fold, (int)(xn && runs > cus ? cus : runs), (int)units, grid, st);
   }
 #undef LAUNCH_CB
   return launched(what);

@@ -412,7 +412,8 @@ def _backward(q, k, v, g, beta, s0, do, dsT, l2norm: bool, q_scale: float, pack=
     """Recompute (prep, unless the forward kept its operands in `r`, and the state pass storing S_c and Vn, unless the
     forward kept them too), the reverse state pass, the per-chunk backward.  Returns (dq, dk, dv in q's dtype; dg,
     dbeta, ds0 float32).  With grouped heads (Hk < H) the per-chunk backward writes dq, dk per value head and
-    macai_gdr_group_sum folds each group (the backward of the repeat the grouped layout replaces).  mixed: bf16 q, k,
+    macai_gdr_group_sum folds each group (the backward of the repeat the grouped layout replaces), or folds them itself
+    (macai_gdr_chunk_bwd_folds; the same bits).  mixed: bf16 q, k,
     v (and dq, dk, dv) with float32 arithmetic, operands and dO (Hk == H)."""
     B, T, H, Hk, DK, DV, NT = _dims(q, v, pack)
     Bc = q.shape[0]
@@ -450,16 +451,19 @@ def _backward(q, k, v, g, beta, s0, do, dsT, l2norm: bool, q_scale: float, pack=
         _launch("state_bwd", "macai_gdr_state_bwd", r["Ke"], r["Qg"], r["W"], r["M"], r["GL"], P(do), P(dsT), dSn, dVn,
                 P(ds0), B, T, H, DK, DV, code, split, *pk, stream)
     CALLS[f"bwd {'reverse' if kept else 'pair' if pair else 'recompute+reverse'} s{split}"] += 1
-    if Hk == H:
+    # two value heads a key head: the kernel sums their dq, dk itself where it runs both in turn
+    fold = Hk != H and bool(N.lib().macai_gdr_chunk_bwd_folds(B, T, H, Hk, DK, DV, code_io, *pk))
+    if Hk == H or fold:
         dqh, dkh = torch.empty_like(q), torch.empty_like(k)
     else:
         dqh = torch.empty(Bc, T, H, DK, device=dev, dtype=dt)
         dkh = torch.empty_like(dqh)
     dv = torch.empty_like(v)
     dg, dbeta = torch.empty_like(g), torch.empty_like(beta)
-    _launch("chunk_bwd", "macai_gdr_chunk_bwd", P(q), P(k), P(v), P(g), P(beta), P(do), r["A"], Sc, dSn, Vn, dVn,
-            P(dqh), P(dkh), P(dv), P(dg), P(dbeta), B, T, H, Hk, DK, DV, code_io, int(l2norm), q_scale, *pk, stream)
-    if Hk == H:
+    _launch("chunk_bwd", "macai_gdr_chunk_bwd_folded" if fold else "macai_gdr_chunk_bwd", P(q), P(k), P(v), P(g), P(beta),
+            P(do), r["A"], Sc, dSn, Vn, dVn, P(dqh), P(dkh), P(dv), P(dg), P(dbeta), B, T, H, Hk, DK, DV, code_io,
+            int(l2norm), q_scale, *pk, stream)
+    if Hk == H or fold:
         return dqh, dkh, dv, dg, dbeta, ds0
     dq, dk = torch.empty_like(q), torch.empty_like(k)
     _launch("group_sum", "macai_gdr_group_sum", P(dqh), P(dq), Bc, T, H, Hk, DK, code, stream)
