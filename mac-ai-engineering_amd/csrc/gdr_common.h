@@ -294,19 +294,22 @@ __device__ __forceinline__ void row_rnorms(float* out, const IT* x, size_t row_b
     if (part == 0) out[r] = (t < T) ? 1.0f / sqrtf(ss + L2_EPS) : 0.f;
   }
 }
-// The same over a bf16 tile already in LDS (row pitch `pitch` elements; rows < nrows, 0 past them).
-template <int D>
+// The same over a bf16 tile already in LDS (row pitch `pitch` elements; rows < nrows, 0 past them).  SW: odd rows hold
+// the 64-byte halves of every 128-byte block swapped (Tile's SW).
+template <int D, bool SW = false>
 __device__ __forceinline__ void row_rnorms_lds(float* out, const bf16* tile, int pitch, int nrows, int nwaves, int w,
                                                int l = lane_id()) {
   const int part = l & 3;
   for (int r0 = 16 * w; r0 < C; r0 += 16 * nwaves) {
     const int r = r0 + (l >> 2);
     const bf16* p = tile + r * pitch + 8 * part;   // rows past nrows hold copies of a valid row: masked below
+    const int flip = SW ? 32 * (r & 1) : 0;
     float ss = 0.f;
 #pragma unroll
     for (int st = 0; st < D / 32; ++st) {
       // two 8-byte reads (rows need only be 8-byte aligned), the same summation order
-      const bf16x4 x0 = *reinterpret_cast<const bf16x4*>(p + 32 * st), x1 = *reinterpret_cast<const bf16x4*>(p + 32 * st + 4);
+      const bf16* ps = p + ((32 * st) ^ flip);
+      const bf16x4 x0 = *reinterpret_cast<const bf16x4*>(ps), x1 = *reinterpret_cast<const bf16x4*>(ps + 4);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float v = (float)(i < 4 ? x0[i] : x1[i - 4]);
