@@ -116,14 +116,15 @@ def make_inputs(cfg, seed, dev, on_device=False, **over):
     return out, c
 
 
-def kernel_costs(B, T, H, DK, DV, es=2, Hk=None, chunks=None, keep=False, segs=1):
+def kernel_costs(B, T, H, DK, DV, es=2, Hk=None, chunks=None, keep=False, segs=1, folds=False):
     """Algorithmic bytes (each declared input read once, each output written once, from argument sizes), split into
     reads and writes, and dense FLOPs (2 per multiply-add, triangular products counted dense) per launch of each
     kernel of the training step.  Hk: key heads of q and k when they come unrepeated (grouped value heads); H by
     default.  chunks: chunks per head over the batch (B ceil(T / 64) by default; packed rows chunk each sequence on
     its own).  keep: the forward's prep also writes A and its state pass S_c and Vn (the stored-states mode: the
     backward then runs neither prep nor the recompute pass).  segs: segments a row's forward runs side by side (the
-    map pass reads W, U, Ke, GL and writes each segment's [A | B]; the scan composes them)."""
+    map pass reads W, U, Ke, GL and writes each segment's [A | B]; the scan composes them).  folds: the per-chunk
+    backward writes dq and dk at the key heads (otherwise per value head, for group_sum to fold)."""
     Hk = Hk or H
     chunks = chunks or B * math.ceil(T / C)
     n = H * chunks                       # chunk-heads
@@ -148,7 +149,7 @@ def kernel_costs(B, T, H, DK, DV, es=2, Hk=None, chunks=None, keep=False, segs=1
         "state_fwd_store": (n * (2 * cdk * es + cdv * 4 + 4), n * (sdk + cdv * es), n * (2 * 2 * C * DK * DV)),
         "state_bwd": (n * (3 * cdk * es + cc * es + 4) + io_v, n * (sdk + cdv * es), state_flops),
         # the per-chunk backward reads q, k, v, g, beta, dO, A, S_c, dS_{c+1}, Vn, dVn; writes dq, dk, dv, dg, dbeta
-        "chunk_bwd": (inp + io_v + n * (cc * es + 2 * sdk + 2 * cdv * es), 2 * io_k + io_v + gb,
+        "chunk_bwd": (inp + io_v + n * (cc * es + 2 * sdk + 2 * cdv * es), 2 * (io_kk if folds else io_k) + io_v + gb,
                       n * (3 * 2 * C * DK * DV + 2 * cc * DK + 3 * 2 * cc * DK + 2 * 2 * cc * DV + 2 * 2 * cc * C
                            + 3 * 2 * cc * DK + 2 * cc * DV)),
         # grouped heads: each of dq, dk folded from per-value-head rows (read H heads, write Hk)
@@ -755,7 +756,9 @@ def main():
     if args.packed:
         cu = kw["cu_seqlens"].tolist()
         chunks = sum(math.ceil((b - a) / C) for a, b in zip(cu, cu[1:]))
-    cost = kernel_costs(B, T, H, DK, DV, Hk=c["Hk"] if args.grouped else None, chunks=chunks, keep=keep)
+    # (the backward sums grouped heads itself at these sizes exactly when the step has no group_sum launch)
+    folds = args.grouped and "group_sum" not in in_step
+    cost = kernel_costs(B, T, H, DK, DV, Hk=c["Hk"] if args.grouped else None, chunks=chunks, keep=keep, folds=folds)
     traffic = measured_traffic(args.config, "stored" if keep else "recompute") if not args.packed else {}
     kernels = {}
     for name, t in in_step.items():
@@ -771,7 +774,8 @@ def main():
             "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": round(bw / HBM_PEAK, 4), "traffic": traffic.get(dom),
             "algorithmic_bytes": cost[dom]["bytes"], "traffic_source": traffic.get("_source")}
     value = tokens / sec
-    other_cost = kernel_costs(B, T, H, DK, DV, Hk=c["Hk"] if args.grouped else None, chunks=chunks, keep=not keep)
+    other_cost = kernel_costs(B, T, H, DK, DV, Hk=c["Hk"] if args.grouped else None, chunks=chunks, keep=not keep,
+                              folds=folds)
     other = {"recompute_prep_in_backward": keep, "ms_per_step": round(sec_other * 1e3, 4),
              "tokens_per_s": round(tokens / sec_other, 1),
              "kernels": {n: {"us": round(t * 1e6, 2), "hbm_frac": round(other_cost[n]["bytes"] / t / HBM_PEAK, 4)}

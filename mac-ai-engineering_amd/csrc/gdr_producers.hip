@@ -170,7 +170,7 @@ constexpr int CV_VE = 4;          // channels a lane
 // input rows at once (the 3 halo rows come again through L2), then forms each output from them.  A wave spans 64
 // consecutive vectors of one block of steps (a wave-uniform start: row addresses are scalar and the ends of the row
 // cost the other waves nothing), a workgroup four consecutive blocks.  Bound by its bytes once the chip is full: at
-// B = 4, T = 1024, C = 6144 in bf16 (101 MB, 18 us at the box's copy rate) 23.0 us, at C = 8192 and T = 2048 (268 MB)
+// B = 4, T = 1024, C = 6144 in bf16 (101 MB, 18 us at the card's copy rate) 23.0 us, at C = 8192 and T = 2048 (268 MB)
 // 49.9 us, 5.4 TB/s.  Lanes of 8 channels (16-byte loads) took 25.0 and 51.5 us (half the waves, twice the registers),
 // 4 or 16 steps 22.9-23.7 and 50.9-52.8; with a correctly rounded division in silu 28.8 and 61 us.
 constexpr int CV_FWD_STEPS = 8;
@@ -238,7 +238,7 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
 // A workgroup is one tile of 64 rows: 64 / S waves, a time block each, over the same 64 vectors, whose sums meet in
 // LDS in wave order (deterministic).  S + 3 rows of du for S of dx: at S = 16 the recomputed rows cost a fifth of the
 // activations.  4-byte x takes twice the registers a row, so it runs S = 8 (all of a lane's loads in flight at 2 waves
-// a SIMD).  Its 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27 us at the box's copy rate and its VALU work is about
+// a SIMD).  Its 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27 us at the card's copy rate and its VALU work is about
 // as long.  Measured there: 36 us, 41 with the taps' gradient (its double sums), against 45 and 65 for the form that
 // staged tiles of x and dy in LDS (three barriers, every row through LDS as float32 twice); at C = 8192, T = 2048 82
 // and 97 against 114 and 154.  S = 8 for bf16 was as fast without the taps' gradient and 14 us slower with it; three
