@@ -161,24 +161,38 @@ __device__ __forceinline__ Frag<MT> cvt(const Frag<float>& x, float s = 1.0f) {
 // prep: G, L, A = (I + L)^-1, W, U, M per chunk
 // ---------------------------------------------------------------------------------------------------------------------
 // 8 waves (two a SIMD, hiding each other's latencies): wave w owns row block w % 4 of the 16 x 16 tiles and every
-// other column block of it from w / 4 on.
-template <typename IT, typename MT, int DK>
-__global__ void __launch_bounds__(512) prep_kernel(PrepArgs a) {
-  // Key features are staged DKS at a time, so the tiles fit LDS at every key width: the products over the key features
-  // accumulate across the passes, and W is formed a pass of columns at a time.  float32 tiles of up to 192 columns
-  // fit in one pass (256: two of 128; 224: seven of 32).
-  constexpr int DKS = (DK <= 192 || sizeof(MT) == 2) ? DK : (DK % 128 == 0 ? 128 : 32);
+// other column block of it from w / 4 on.  Bound by latency: a chunk-head is a chain of short phases between barriers
+// (loads, products, a serial substitution on one wave, block products, stores), so L and A lie where the key tile was
+// and V^T where K^'s transpose was, and two workgroups share a CU up to key widths of 128 (73 KB each; 106 KB with
+// tiles of their own, one a CU).  At 512 chunk-heads of 128 x 128 in float32 61 -> 47 us, with A's fragments kept out
+// of scratch 40 (125-133 MB, 3.2 TB/s; its float32 MFMAs are 15).
+// Key features are staged DKS at a time, so the tiles fit LDS at every key width: the products over the key features
+// accumulate across the passes, and W is formed a pass of columns at a time.  float32 tiles of up to 192 columns fit in
+// one pass (256: two of 128; 224: seven of 32).
+template <typename MT, int DK>
+struct PrepLds {
+  static constexpr int DKS = (DK <= 192 || sizeof(MT) == 2) ? DK : (DK % 128 == 0 ? 128 : 32);
   static_assert(DK % DKS == 0 && DKS % 32 == 0, "prep key-column passes");
-  constexpr int NPASS = DK / DKS;
-  constexpr int KP = DKS + 8;  // pitch of [C][DKS] tiles (elements)
-  constexpr int CP = C + 8;    // pitch of [*][C] MT tiles
-  constexpr int FP = C + 4;    // pitch of fp32 [C][C] tiles
-  constexpr int QSZ = (C * KP > DKS * CP) ? C * KP : DKS * CP;
-  constexpr int KSZ = (C * KP > C * CP) ? C * KP : C * CP;
-  __shared__ __attribute__((aligned(16))) MT sK[KSZ];    // K^ rows (a pass of columns); then (beta V)^T blocks
-  __shared__ __attribute__((aligned(16))) MT sQ[QSZ];    // Q^ rows (a pass); then (beta gamma K^)^T (a pass)
-  __shared__ __attribute__((aligned(16))) float sL[C * FP];
-  __shared__ __attribute__((aligned(16))) float sA[C * FP];
+  static constexpr int KP = DKS + 8;  // pitch of [C][DKS] tiles (elements)
+  static constexpr int CP = C + 8;    // pitch of [*][C] MT tiles
+  static constexpr int FP = C + 4;    // pitch of fp32 [C][C] tiles
+  static constexpr int QN = (C * KP > DKS * CP) ? C * KP : DKS * CP;
+  static constexpr int QSZ = (QN > C * CP) ? QN : C * CP;
+  static constexpr int VB = (QSZ >= 128 * CP) ? 128 : 64;          // value columns of (beta V)^T a stage
+  static constexpr int LA = 2 * C * FP * 4;                        // bytes of L and A
+  static constexpr int KSZ = (C * KP * (int)sizeof(MT) > LA) ? C * KP : LA / (int)sizeof(MT);
+  // two workgroups a CU where two fit its 160 KB (with 3 KB of scalars each): four waves a SIMD
+  static constexpr int WAVES = ((KSZ + QSZ) * (int)sizeof(MT) + 3072 <= 80 * 1024) ? 4 : 2;
+};
+
+template <typename IT, typename MT, int DK>
+__global__ void __launch_bounds__(512, (PrepLds<MT, DK>::WAVES)) prep_kernel(PrepArgs a) {
+  using LD = PrepLds<MT, DK>;
+  constexpr int DKS = LD::DKS, NPASS = DK / DKS, KP = LD::KP, CP = LD::CP, FP = LD::FP;
+  __shared__ __attribute__((aligned(16))) MT sK[LD::KSZ];   // K^ rows (a pass of columns); then L and A
+  __shared__ __attribute__((aligned(16))) MT sQ[LD::QSZ];   // Q^ rows; then (beta gamma K^)^T (a pass each); (beta V)^T
+  float* const sL = (float*)sK;
+  float* const sA = sL + C * FP;
   __shared__ ChunkScalars cs;
   __shared__ float rk[C], rq[C];
 
@@ -272,6 +286,7 @@ __global__ void __launch_bounds__(512) prep_kernel(PrepArgs a) {
       }
     }
   }
+  __syncthreads();                         // the products are done with sK, where L and A go
   // L (strictly lower, fp32) into LDS; M out
   {
     const int mi = rb;
@@ -363,21 +378,25 @@ __global__ void __launch_bounds__(512) prep_kernel(PrepArgs a) {
       }
       for (int ni = half; ni < DKS / 16; ni += 2) {
         f4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < np; ++p) mma(acc, af[p], frag_k_raw(sQ, CP, 16 * ni, 32 * p));
+#pragma unroll
+        for (int p = 0; p < 2; ++p)        // (unrolled: at four waves a SIMD an indexed af[p] lives in scratch)
+          if (p < np) mma(acc, af[p], frag_k_raw(sQ, CP, 16 * ni, 32 * p));
 #pragma unroll
         for (int r = 0; r < 4; ++r) Wc[(16 * rb + 4 * j + r) * DK + ps * DKS + 16 * ni + (l & 15)] = from_f<MT>(acc[r]);
       }
     }
-    // U = A (beta V), 64 value columns at a time staged transposed in sK
+    // U = A (beta V), VB value columns at a time staged transposed in sQ
     float* Uc = a.U + bhc * C * DV;
-    for (int vb = 0; vb < DV; vb += 64) {
-      const int nv = (DV - vb < 64) ? DV - vb : 64;
+    for (int vb = 0; vb < DV; vb += LD::VB) {
+      const int nv = (DV - vb < LD::VB) ? DV - vb : LD::VB;
       __syncthreads();
-      stage_rows_T<MT, IT>(sK, CP, v + vb, v_pitch, t0, T, nv, [&](int r) { return cs.beta[r]; });
+      stage_rows_T<MT, IT>(sQ, CP, v + vb, v_pitch, t0, T, nv, [&](int r) { return cs.beta[r]; });
       __syncthreads();
       for (int ni = half; ni < nv / 16; ni += 2) {
         f4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int p = 0; p < np; ++p) mma(acc, af[p], frag_k_raw(sK, CP, 16 * ni, 32 * p));
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+          if (p < np) mma(acc, af[p], frag_k_raw(sQ, CP, 16 * ni, 32 * p));
 #pragma unroll
         for (int r = 0; r < 4; ++r) Uc[(16 * rb + 4 * j + r) * DV + vb + 16 * ni + (l & 15)] = acc[r];
       }
