@@ -1696,9 +1696,10 @@ struct StateBwdLds {
       DIRECT ? 0 : Buffers<SZ * (int)sizeof(MT), (STG + SCAL + EX) * (int)sizeof(MT) + TOUCH_SINK>::N;
   static constexpr int O_STG = NBUF * SZ, O_SCAL = O_STG + STG, O_EX = O_SCAL + SCAL;
   static constexpr int ELEMS = O_EX + EX;
-  // see StateFwdLds::KS_OK and PHASED
+  // see StateFwdLds::KS_OK and PHASED; of one column slice only: at two (5 waves, 256 registers each) the phased pass
+  // spills, 396 us against 143 at 64 head-rows of 16 chunks
   static constexpr bool KS_OK = KS == 2 && sizeof(MT) == 4 && (DK == 64 || DK == 128) && !DIRECT && NW <= 2;
-  static constexpr bool PHASED = KS_OK && NBUF == 1;
+  static constexpr bool PHASED = KS_OK && NBUF == 1 && NW == 1;
 };
 
 // The key-split float32 reverse pass (the compute waves of state_bwd_body with KS = 2; see state_fwd_ks): wave

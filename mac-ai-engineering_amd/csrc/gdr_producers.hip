@@ -145,7 +145,8 @@ __device__ __forceinline__ float tap_dot(const float (&tw)[CV_TAPS][N], int i, f
   }
 }
 // 1 / d for d >= 1 (or NaN): the hardware reciprocal (1 ulp) and one Newton step, r + r (1 - d r), which rounds as the
-// division does but for rare ties (d held finite, so that an overflowed exponential still gives 0).  The division took a
+// division does but for rare ties (d held finite, so that an overflowed exponential still gives 0: the instruction flushes
+// subnormal results).  The division took a
 // fifth of the backward's instructions; the results' errors against float64 are the same to four digits.
 __device__ __forceinline__ float recip(float d) {
   d = fminf(d, 3.0e38f);

@@ -55,3 +55,33 @@ def test_gates_rows_and_heads(rows, H, dtype, ptypes):
     xs = [_draw((rows, H), dtype, gen), _draw((rows, H), dtype, gen, 3.0), _draw((H,), ptypes[0], gen),
           _draw((H,), ptypes[1], gen)]
     _compare(gates, P.gates, xs, gen)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_conv_infinities_and_nan(dtype):
+    """Infinite and NaN inputs, and ones whose exponential overflows: y and dx are finite, infinite or NaN where plain
+    PyTorch's are, of the same sign."""
+    print("case conv infinities", dtype, flush=True)
+    T, C = 41, 24
+    gen = torch.Generator().manual_seed(5)
+    x, w = _draw((1, T, C), dtype, gen), _draw((C, 1, 4), dtype, gen, 0.3).abs()
+    for i, bad in enumerate((float("inf"), float("-inf"), float("nan"), 3e4, -3e4, 600.0, -600.0)):
+        x[0, 6 * i, i::7] = bad
+    leaf = x.cuda().requires_grad_(True)
+    got = conv_qkv(leaf, w.cuda(), 8, 8, 1, 8, False, dtype)
+    ups = [_draw(o.shape, dtype, gen) for o in got]
+    dx, = torch.autograd.grad(got, leaf, [u.cuda() for u in ups])
+    # in float32 on the CPU, sigmoid as 1 / (1 + exp(-u)); a window holds one such value at most
+    x32, w32 = torch.nn.functional.pad(x.float(), (0, 0, 3, 0)), w.float().reshape(C, 4)
+    u = sum(w32[:, j] * x32[:, j:j + T] for j in range(4))
+    s = 1 / (1 + torch.exp(-u))
+    y = u * s
+    du = torch.nn.functional.pad(torch.cat(ups, 2).reshape(1, T, C).float() * (s * (1 + u * (1 - s))), (0, 0, 0, 3))
+    want = [y.reshape(T, C), sum(w32[:, 3 - j] * du[:, j:j + T] for j in range(4)).reshape(T, C)]
+    want = [t.to(dtype) for t in want]
+    have = [torch.cat([o.detach().cpu().reshape(T, 8) for o in got], 1), dx.cpu().reshape(T, C)]
+    for name, a, b in zip(("y", "dx"), have, want):
+        for what, fa, fb in (("nan", a.isnan(), b.isnan()), ("inf", a.isinf(), b.isinf())):
+            assert torch.equal(fa, fb), (name, what, (fa != fb).nonzero()[:8].tolist())
+        inf = b.isinf()
+        assert torch.equal(a[inf] > 0, b[inf] > 0), name
