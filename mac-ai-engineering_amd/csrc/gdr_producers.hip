@@ -7,7 +7,7 @@
 //
 // The convolution is an HBM stream: every input and output byte crosses once (the 3-row halos come again through L2).
 // A lane owns a channel vector over consecutive time steps, all its input rows loaded at once, a wave 64 consecutive
-// vectors: 4 channels over 8 steps in the forward (conv_fwd_kernel), over 16 or 8 in the backward (conv_bwd_kernel),
+// vectors: 4 channels over 8 steps in the forward (conv_fwd_kernel), 8 bytes over 16 in the backward (conv_bwd_kernel),
 // which forms du = dy silu'(u) for its steps and the 3 after them in registers, dx from du's
 // windows (one writer an element) and the taps' gradient's sums over its steps; a tile of 64 rows adds its waves' sums
 // in order through LDS, sum_columns_kernel the tiles' partials in tile order: deterministic.
@@ -230,24 +230,27 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
   }
 }
 
-// The backward, like the forward, streams: a lane owns 4 channels over S consecutive time steps t0 .. t0 + S - 1 and
-// issues all its loads at once -- x[t0 - 3 .. t0 + S + 2] and the upstream gradient dy[t0 .. t0 + S + 2] (q's and k's
-// copies summed in copy order) -- then walks the rows with everything in registers:
+// The backward, like the forward, streams: a lane owns 4 channels (2 of 4-byte x) over S consecutive time steps
+// t0 .. t0 + S - 1 and issues all its loads at once -- x[t0 - 3 .. t0 + S + 2] and the upstream gradient
+// dy[t0 .. t0 + S + 2] (q's and k's copies summed in copy order) -- then walks the rows with everything in registers:
 //   du[t] = dy s (1 + u (1 - s)), s = sigmoid(u)   (0 past the end), for its S rows and the 3 after them,
 //   dx[t] = w0 du[t + 3] + w1 du[t + 2] + w2 du[t + 1] + w3 du[t],
 //   part[tile][c, j] = sum over the tile's t of du[t] x[t - 3 + j], in double.
 // A workgroup is one tile of 64 rows: 64 / S waves, a time block each, over the same 64 vectors, whose sums meet in
 // LDS in wave order (deterministic).  S + 3 rows of du for S of dx: at S = 16 the recomputed rows cost a fifth of the
-// activations.  4-byte x takes twice the registers a row, so it runs S = 8 (all of a lane's loads in flight at 2 waves
-// a SIMD).  Its 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27 us at the card's copy rate and its VALU work is about
+// activations.  4-byte x takes 2 channels a lane, the same bytes: 4 spill at S = 16, and at S = 8 (half as many rows
+// recomputed again) took 92 us against 66 at B = 4, T = 1024, C = 6144 and 142 against 99 at C = 8192 with repeated
+// heads (the LDS form below 80 and 119).  All of a lane's loads are in flight at 2 waves
+// a SIMD.  Its 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27 us at the card's copy rate and its VALU work is about
 // as long.  Measured there: 36 us, 41 with the taps' gradient (its double sums), against 45 and 65 for the form that
 // staged tiles of x and dy in LDS (three barriers, every row through LDS as float32 twice); at C = 8192, T = 2048 82
 // and 97 against 114 and 154.  S = 8 for bf16 was as fast without the taps' gradient and 14 us slower with it; three
 // waves a SIMD spills.
-template <typename T> constexpr int conv_bwd_steps() { return sizeof(T) == 4 ? 8 : 16; }
+constexpr int CV_BWD_STEPS = 16;
+template <typename T> constexpr int conv_bwd_vec() { return sizeof(T) == 4 ? 2 : CV_VE; }
 template <typename T, typename TV, bool TAPS>
-__global__ void __launch_bounds__(64 * (CV_ROWS / conv_bwd_steps<T>()), 2) conv_bwd_kernel(ConvArgs a) {
-  constexpr int VE = CV_VE, S = conv_bwd_steps<T>(), NWAVE = CV_ROWS / S;
+__global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_kernel(ConvArgs a) {
+  constexpr int VE = conv_bwd_vec<T>(), S = CV_BWD_STEPS, NWAVE = CV_ROWS / S;
   constexpr bool EXACT = sizeof(T) == 4;
   constexpr int XR = S + 2 * CV_HALO, DR = S + CV_HALO;
   __shared__ double red[TAPS ? NWAVE : 1][TAPS ? VE : 1][64];   // one tap's sums: a row a wave
@@ -662,9 +665,10 @@ int macai_gdr_conv_bwd_typed(const void* x, const float* w, const void* dq, cons
   ConvArgs a{x, w, nullptr, nullptr, nullptr, nullptr, dq, dk, dv, dx, dwp, (int)B, (int)T, (int)C, (int)KD, (int)DK,
              (int)REP, ntiles, MACAI_GDR_F32};
   hipStream_t st = (hipStream_t)stream;
-  // 64 vectors of CV_VE channels by a tile of CV_ROWS steps; a wave a block of conv_bwd_steps of them
-  const dim3 grid((unsigned)((C + 64 * CV_VE - 1) / (64 * CV_VE)), (unsigned)ntiles, (unsigned)B);
-  const dim3 block(64 * (CV_ROWS / (dtype == MACAI_GDR_F32 ? conv_bwd_steps<float>() : conv_bwd_steps<bf16>())));
+  // 64 vectors of conv_bwd_vec channels by a tile of CV_ROWS steps; a wave a block of CV_BWD_STEPS of them
+  const int64_t span = 64 * (dtype == MACAI_GDR_F32 ? conv_bwd_vec<float>() : conv_bwd_vec<bf16>());
+  const dim3 grid((unsigned)((C + span - 1) / span), (unsigned)ntiles, (unsigned)B);
+  const dim3 block(64 * (CV_ROWS / CV_BWD_STEPS));
   if (dwp) {
     DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_kernel<PT, PV, true>), grid, block, 0, st, a)))
   } else {
