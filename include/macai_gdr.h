@@ -204,8 +204,9 @@ int macai_gdr_group_sum(const void* x, void* y, int64_t B, int64_t T, int64_t H,
  * u[t, c] = sum_j w[c, j] x[t - 3 + j, c] (zero before the start, float32), y = u sigmoid(u) rounded once; q, k =
  * the first two KD-channel blocks as [B, T, KD / DK * REP, DK] in x's dtype, each key head written REP times
  * (REP = 1: key heads only, the layout the rule reads natively; REP = value heads / key heads: transformers' repeat),
- * v = the last VD channels as [B, T, VD / DV, DV] in vdtype.  dtype, vdtype: F32, BF16 or F16.  Replaces the
- * reference's conv_fwd kernel launch (layer/_conv.py:191-193; kernel 1-24, 47-82). */
+ * v = the last VD channels as [B, T, VD / DV, DV] in vdtype.  dtype, vdtype: F32, BF16 or F16.  For float32 x the
+ * quotient u / (1 + e^-u) is a rounded division; for 2-byte x, here and in the backward, u times a refined hardware
+ * reciprocal, which differs from the division's in rare ties only.  Replaces the reference's conv_fwd kernel launch (layer/_conv.py:191-193; kernel 1-24, 47-82). */
 int macai_gdr_conv_fwd(const void* x, const float* w, void* q, void* k, void* v, int64_t B, int64_t T, int64_t C,
                        int64_t KD, int64_t DK, int64_t REP, int64_t DV, int32_t dtype, int32_t vdtype, void* stream);
 

@@ -144,26 +144,27 @@ __device__ __forceinline__ float tap_dot(const float (&tw)[CV_TAPS][N], int i, f
     return fmaf(tw[0][i], w0, fmaf(tw[1][i], w1, fmaf(tw[2][i], w2, tw[3][i] * w3)));
   }
 }
-// 1 / d for d >= 1 (or NaN): the hardware reciprocal (1 ulp) and one Newton step, r + r (1 - d r), which rounds as the
-// division does but for rare ties (d held finite, so that an overflowed exponential still gives 0: the instruction flushes
-// subnormal results).  The division took a
-// fifth of the backward's instructions; the results' errors against float64 are the same to four digits.
-__device__ __forceinline__ float recip(float d) {
-  d = fminf(d, 3.0e38f);
+// 1 / (1 + e) for e >= 0 (or NaN): the hardware reciprocal (1 ulp) and one Newton step, r + r (1 - d r), which rounds as
+// the division does but for rare ties.  Formed at 1/16 of the scale: the instruction flushes subnormal results, and past
+// e = 2^126 (u below -87.3) the quotient is one while u times it is not.  d is held finite, so an overflowed exponential
+// still gives 0.  The division took a fifth of the backward's instructions; the results' errors against float64 are the
+// same to four digits.
+__device__ __forceinline__ float recip1p(float e) {
+  const float d = fminf(fmaf(0.0625f, e, 0.0625f), 3.0e38f);
   const float r = __builtin_amdgcn_rcpf(d);
-  return fmaf(fmaf(-d, r, 1.0f), r, r);
+  return 0.0625f * fmaf(fmaf(-d, r, 1.0f), r, r);
 }
 template <bool EXACT>
 __device__ __forceinline__ float logistic(float u) {
   if constexpr (EXACT) return 1.0f / (1.0f + expf(-u));
-  else return recip(1.0f + __expf(-u));
+  else return recip1p(__expf(-u));
 }
 // u sigmoid(u) with one rounding after the exponential for float32 inputs (a division, not u times a rounded
 // reciprocal, whose two roundings put the float32 output past twice PyTorch's silu error)
 template <bool EXACT>
 __device__ __forceinline__ float silu(float u) {
   if constexpr (EXACT) return u / (1.0f + expf(-u));
-  else return u * recip(1.0f + __expf(-u));
+  else return u * recip1p(__expf(-u));
 }
 
 constexpr int CV_VE = 4;          // channels a lane

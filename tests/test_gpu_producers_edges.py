@@ -85,3 +85,26 @@ def test_conv_infinities_and_nan(dtype):
             assert torch.equal(fa, fb), (name, what, (fa != fb).nonzero()[:8].tolist())
         inf = b.isinf()
         assert torch.equal(a[inf] > 0, b[inf] > 0), name
+
+
+def test_conv_far_negative():
+    """u between -88.7 and -87.3, where 1 / (1 + e^-u) is subnormal and u times it is not: y and dx keep their values
+    (around -1e-36), in the type's precision and that of the exponential (|u| 2^-24 of its argument's rounding, four
+    times over)."""
+    print("case conv far negative", flush=True)
+    us = torch.tensor([-87.0, -87.5, -88.0, -88.5])
+    T, C = us.numel(), 24
+    x = us.view(1, T, 1).expand(1, T, C).contiguous()
+    w = torch.zeros(C, 1, 4)
+    w[..., 3] = 1.0                                   # y[t] = silu(x[t])
+    u64 = x.double().requires_grad_(True)
+    want = u64 * torch.sigmoid(u64)
+    dwant, = torch.autograd.grad(want, u64, torch.ones_like(want))
+    for v_dtype in (torch.bfloat16, torch.float32):
+        leaf = x.bfloat16().cuda().requires_grad_(True)
+        out = conv_qkv(leaf, w.cuda(), 8, 8, 1, 8, False, v_dtype)
+        dx, = torch.autograd.grad(out, leaf, [torch.ones_like(o) for o in out])
+        parts = want.detach().reshape(T, 3, 8).unbind(1)
+        for o, r in [*zip((o.reshape(T, 8) for o in out), parts), (dx.reshape(T, C), dwant.reshape(T, C))]:
+            e = ((o.detach().cpu().double() - r) / r).abs().max().item()
+            assert e < 2.0 ** -BITS[o.dtype] + 4 * 89 * 2.0 ** -24, (v_dtype, o.dtype, e)
