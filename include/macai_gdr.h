@@ -206,7 +206,8 @@ int macai_gdr_group_sum(const void* x, void* y, int64_t B, int64_t T, int64_t H,
  * (REP = 1: key heads only, the layout the rule reads natively; REP = value heads / key heads: transformers' repeat),
  * v = the last VD channels as [B, T, VD / DV, DV] in vdtype.  dtype, vdtype: F32, BF16 or F16.  For float32 x the
  * quotient u / (1 + e^-u) is a rounded division; for 2-byte x, here and in the backward, u times a refined hardware
- * reciprocal, which differs from the division's in rare ties only.  Replaces the reference's conv_fwd kernel launch (layer/_conv.py:191-193; kernel 1-24, 47-82). */
+ * reciprocal, which differs from the division's in rare ties only.  Replaces the reference's conv_fwd kernel launch
+ * (layer/_conv.py:191-193; kernel 1-24, 47-82). */
 int macai_gdr_conv_fwd(const void* x, const float* w, void* q, void* k, void* v, int64_t B, int64_t T, int64_t C,
                        int64_t KD, int64_t DK, int64_t REP, int64_t DV, int32_t dtype, int32_t vdtype, void* stream);
 
@@ -248,9 +249,9 @@ int macai_gdr_gates_bwd(const void* b, const void* a, const float* A_log, const 
 
 /* The two entry points above with A_log and dt_bias in their own types (codes atype, dtype_bias: F32, BF16 or F16).  The
  * forward writes their float32 copies [2, H] to params when it is non-NULL (what the backward takes).  The backward
- * always writes dA_log and ddt_bias, in those types: its one pass forms its workgroups' sums in part, double
- * [macai_gdr_gates_partials(n, H)] scratch, and a second launch adds them in a fixed order, where macai_gdr_gates_bwd
- * without scratch runs a pass of one workgroup a head. */
+ * always writes dA_log and ddt_bias, in those types: over many rows its pass forms its workgroups' sums in part, double
+ * [macai_gdr_gates_partials(n, H)] scratch, and a second launch adds them in a fixed order; over few rows, and always in
+ * macai_gdr_gates_bwd, which has no scratch, a pass of one workgroup a head forms them. */
 int macai_gdr_gates_fwd_typed(const void* b, const void* a, const void* A_log, int32_t atype, const void* dt_bias,
                               int32_t dtype_bias, float* params, float* beta, float* g, int64_t n, int64_t H,
                               int32_t dtype, void* stream);

@@ -11,8 +11,9 @@
 // which forms du = dy silu'(u) for its steps and the 3 after them in registers, dx from du's
 // windows (one writer an element) and the taps' gradient's sums over its steps; a tile of 64 rows adds its waves' sums
 // in order through LDS, sum_columns_kernel the tiles' partials in tile order: deterministic.
-// The gates are one pass each way, an element a lane; the backward's also forms its workgroup's sums of A_log's and
-// dt_bias's gradients, which a second launch adds in a fixed tree.
+// The gates are one pass each way, an element a lane; over many rows the backward's also forms its workgroups' sums of
+// A_log's and dt_bias's gradients, which a second launch adds in a fixed order, over few a second pass takes a workgroup a
+// head (gate_direct_rows).
 #include <hip/hip_runtime.h>
 
 #include "gdr_abi.h"
@@ -430,86 +431,97 @@ __device__ __forceinline__ double softplus_t20(double x) { return x > 20.0 ? x :
 __device__ __forceinline__ double softplus_t20_grad(double x) { return x > 20.0 ? 1.0 : 1.0 / (1.0 + exp(-x)); }
 
 // The gates move under a megabyte per layer, so they are bound by latency, not bandwidth: one element a lane, so
-// that a layer's elements spread over every lane of the chip and each lane runs one exponential chain.  A_log and
-// dt_bias are read in the types of codes pt[0], pt[1]; with `params` non-null the first lanes write their float32
-// copies ([2, H]) there.
+// that a layer's elements spread over every lane of the chip and each lane runs one exponential chain.  TYPED: A_log and
+// dt_bias are read in the types of codes ta, td, and with `params` non-null the first lanes write their float32 copies
+// ([2, H]) there; otherwise both are float32 (the branches on the codes cost 0.1 us of 2.4).
 constexpr int GATE_THREADS = 256;
 struct GateParams {
   const void *alog, *dtb;
   int ta, td;                                // dtype codes
-  __device__ __forceinline__ float a(int h) const { return load_code(alog, ta, h); }
-  __device__ __forceinline__ float d(int h) const { return load_code(dtb, td, h); }
 };
-template <typename T>
+template <typename T, bool TYPED>
 __global__ void __launch_bounds__(GATE_THREADS) gates_fwd_kernel(const T* b, const T* a, GateParams p, float* params,
                                                                  float* beta, float* g, int64_t n, int H) {
   const int64_t i = (int64_t)blockIdx.x * GATE_THREADS + threadIdx.x;
   if (i >= n) return;
   const int head = (int)(i % H);             // heads run fastest: element i is head i mod H
-  const float alog = p.a(head), dtb = p.d(head);
-  if (params && i < H) {                     // n is a multiple of H
-    params[i] = alog;
-    params[H + i] = dtb;
+  float alog, dtb;
+  if constexpr (TYPED) {
+    alog = load_code(p.alog, p.ta, head);
+    dtb = load_code(p.dtb, p.td, head);
+    if (params && i < H) {                   // n is a multiple of H
+      params[i] = alog;
+      params[H + i] = dtb;
+    }
+  } else {
+    alog = ((const float*)p.alog)[head];
+    dtb = ((const float*)p.dtb)[head];
   }
   const double rate = -exp((double)alog);
   beta[i] = (float)(1.0 / (1.0 + exp(-(double)(float)b[i])));
   g[i] = (float)(rate * softplus_t20((double)(float)a[i] + (double)dtb));
 }
 
-// db = dbeta s (1 - s), s = sigmoid(b); da = dg (-exp(A_log)) softplus'(a + dt_bias).  PARTS: also each workgroup's
-// sums, per head, of the parameters' gradients' terms (dA_log: dg g; ddt_bias: da before its rounding), in double, to
-// part[workgroup][2][H].  A workgroup's elements go by whole rows of H heads: thread i of it takes head i % H of row
-// i / H and then every rpp-th row (rpp = 256 / H rows at once; heads past 256 in further passes), its own sums in row
-// order, and the rpp sums of a head add in order through LDS: deterministic.  gates_params_kernel adds the workgroups'
-// in order.  Bound by the chain of double exponentials, so it is spread over every CU: at B T = 4096, H = 16 in bf16
-// 6.0 us with the sums and 3.8 for gates_params_kernel, where this pass without them (3.5) and one of one workgroup a
-// head (14.8: two exponentials and a logarithm an element on H CUs) took 18.3.
-template <typename T, bool PARTS>
+// db = dbeta s (1 - s), s = sigmoid(b); da = dg (-exp(A_log)) softplus'(a + dt_bias).
+template <typename T>
 __global__ void __launch_bounds__(GATE_THREADS) gates_bwd_kernel(const T* b, const T* a, const float* alog,
                                                                  const float* dtb, const float* dbeta,
-                                                                 const float* dg, T* db, T* da, double* part,
-                                                                 int64_t rows, int H, int per) {
-  __shared__ double red[PARTS ? 2 : 1][PARTS ? GATE_THREADS : 1];
-  const int64_t r0 = (int64_t)blockIdx.x * per, r1 = r0 + per < rows ? r0 + per : rows;
+                                                                 const float* dg, T* db, T* da, int64_t n, int H) {
+  const int64_t i = (int64_t)blockIdx.x * GATE_THREADS + threadIdx.x;
+  if (i >= n) return;
+  const int head = (int)(i % H);
+  const double rate = -exp((double)alog[head]);
+  const double sig = 1.0 / (1.0 + exp(-(double)(float)b[i]));
+  db[i] = (T)(float)((double)dbeta[i] * (sig - sig * sig));          // d sigmoid = s (1 - s)
+  da[i] = (T)(float)((double)dg[i] * rate * softplus_t20_grad((double)(float)a[i] + (double)dtb[head]));
+}
+
+// The same pass with each workgroup's sums, per head, of the parameters' gradients' terms (dA_log: dg g; ddt_bias: da
+// before its rounding), in double, to part[group][2][H].  A workgroup takes `per` whole rows of min(H, 256) heads
+// (block % hblocks says which heads): thread i takes head i % H of row i / H and then every rpp-th row (rpp = 256 / H
+// rows at once), its own sums in row order, and the rpp sums of a head add in order through LDS: deterministic.
+// gates_params_kernel adds the groups' in order.  Bound by the chain of double exponentials, so it is spread over every
+// CU: see gate_direct_rows for what it is measured against.
+template <typename T>
+__global__ void __launch_bounds__(GATE_THREADS) gates_bwd_sums_kernel(const T* b, const T* a, const float* alog,
+                                                                      const float* dtb, const float* dbeta,
+                                                                      const float* dg, T* db, T* da, double* part,
+                                                                      int64_t rows, int H, int per, int hblocks) {
+  __shared__ double red[2][GATE_THREADS];
+  const int64_t group = blockIdx.x / hblocks;
+  const int64_t r0 = group * per, r1 = r0 + per < rows ? r0 + per : rows;
   const int rpp = H < GATE_THREADS ? GATE_THREADS / H : 1;   // rows at once
   const int sub = H < GATE_THREADS ? threadIdx.x / H : 0;
-  for (int h0 = 0; h0 < H; h0 += GATE_THREADS) {
-    const int h = H < GATE_THREADS ? threadIdx.x % H : h0 + threadIdx.x;
-    double s_a = 0.0, s_d = 0.0;
-    if (sub < rpp && h < H) {
-      const double rate = -exp((double)alog[h]), bias = (double)dtb[h];
-      for (int64_t r = r0 + sub; r < r1; r += rpp) {
-        const int64_t i = r * H + h;
-        const double sig = 1.0 / (1.0 + exp(-(double)(float)b[i]));
-        db[i] = (T)(float)((double)dbeta[i] * (sig - sig * sig));          // d sigmoid = s (1 - s)
-        const double x = (double)(float)a[i] + bias, gr = (double)dg[i] * rate, dx = gr * softplus_t20_grad(x);
-        da[i] = (T)(float)dx;
-        if (PARTS) {
-          s_a = fma(gr, softplus_t20(x), s_a);
-          s_d += dx;
-        }
-      }
+  const int h = H < GATE_THREADS ? threadIdx.x % H : blockIdx.x % hblocks * GATE_THREADS + threadIdx.x;
+  double s_a = 0.0, s_d = 0.0;
+  if (sub < rpp && h < H) {
+    const double rate = -exp((double)alog[h]), bias = (double)dtb[h];
+    for (int64_t r = r0 + sub; r < r1; r += rpp) {
+      const int64_t i = r * H + h;
+      const double sig = 1.0 / (1.0 + exp(-(double)(float)b[i]));
+      db[i] = (T)(float)((double)dbeta[i] * (sig - sig * sig));
+      const double x = (double)(float)a[i] + bias, gr = (double)dg[i] * rate, dx = gr * softplus_t20_grad(x);
+      da[i] = (T)(float)dx;
+      s_a = fma(gr, softplus_t20(x), s_a);
+      s_d += dx;
     }
-    if constexpr (PARTS) {
-      if (h0) __syncthreads();               // the previous heads' sums are read
-      red[0][threadIdx.x] = s_a;
-      red[1][threadIdx.x] = s_d;
-      __syncthreads();
-      if (sub == 0 && h < H) {
-        for (int k = 1; k < rpp; ++k) {
-          s_a += red[0][k * H + h];
-          s_d += red[1][k * H + h];
-        }
-        double* out = part + (size_t)blockIdx.x * 2 * H;
-        out[h] = s_a;
-        out[H + h] = s_d;
-      }
+  }
+  red[0][threadIdx.x] = s_a;
+  red[1][threadIdx.x] = s_d;
+  __syncthreads();
+  if (sub == 0 && h < H) {
+    for (int k = 1; k < rpp; ++k) {
+      s_a += red[0][k * H + h];
+      s_d += red[1][k * H + h];
     }
+    double* out = part + (size_t)group * 2 * H;
+    out[h] = s_a;
+    out[H + h] = s_d;
   }
 }
 
-// dA_log[h] and ddt_bias[h]: the workgroups' sums of gates_bwd_kernel added in double, rounded to float32 and then to
-// the gradients' types.  A wave a head: lane l adds workgroups l, l + 64, ... in order, then the lanes add by a fixed
+// dA_log[h] and ddt_bias[h]: the groups' sums of gates_bwd_sums_kernel added in double, rounded to float32 and then to
+// the gradients' types.  A wave a head: lane l adds groups l, l + 64, ... in order, then the lanes add by a fixed
 // butterfly.
 __global__ void __launch_bounds__(64) gates_params_kernel(const double* part, void* dA, void* ddt, int ta, int td,
                                                           int groups, int H) {
@@ -530,13 +542,14 @@ __global__ void __launch_bounds__(64) gates_params_kernel(const double* part, vo
   }
 }
 
-// The parameters' gradients for callers without scratch: one workgroup a head; thread i takes rows i, i + 256, ... in
-// order, then a wave sums its lanes by a fixed butterfly and the four waves add in order.  Deterministic.  Terms and
-// sums in double, rounded once: a head's rows of dg carry both signs, so the sums can cancel.
+// The parameters' gradients without scratch, beside gates_bwd_kernel: one workgroup a head; thread i takes rows i,
+// i + 256, ... in order, then a wave sums its lanes by a fixed butterfly and the four waves add in order.
+// Deterministic.  Terms and sums in double, rounded to float32 and then to the gradients' types: a head's rows of dg
+// carry both signs, so the sums can cancel.
 template <typename T>
 __global__ void __launch_bounds__(256) gates_params_direct_kernel(const T* a, const float* alog, const float* dtb,
-                                                                  const float* dg, float* dA, float* ddt, int64_t rows,
-                                                                  int H) {
+                                                                  const float* dg, void* dA, void* ddt, int ta, int td,
+                                                                  int64_t rows, int H) {
   const int h = blockIdx.x;
   const double rate = -exp((double)alog[h]), bias = (double)dtb[h];
   double s_a = 0.0, s_d = 0.0;
@@ -558,8 +571,8 @@ __global__ void __launch_bounds__(256) gates_params_direct_kernel(const T* a, co
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    dA[h] = (float)(((wa[0] + wa[1]) + wa[2]) + wa[3]);
-    ddt[h] = (float)(((wd[0] + wd[1]) + wd[2]) + wd[3]);
+    store_code(dA, ta, h, (float)(((wa[0] + wa[1]) + wa[2]) + wa[3]));
+    store_code(ddt, td, h, (float)(((wd[0] + wd[1]) + wd[2]) + wd[3]));
   }
 }
 
@@ -591,8 +604,15 @@ int check_conv(const char* what, int64_t B, int64_t T, int64_t C, int64_t KD, in
   return MACAI_GDR_OK;
 }
 
-// The gates' backward's workgroups for `rows` rows of H heads, `per` rows each: one pass of rows a workgroup (an element
-// a lane) up to 512 workgroups, then as many passes as keep to that (the second stage adds the workgroups' sums).
+// Up to this many rows the parameters' gradients come from gates_params_direct_kernel (a workgroup a head), whose
+// chain is then the shorter one; past them from gates_bwd_sums_kernel and gates_params_kernel.  Where the two cross, with
+// the pass over the elements in each, at H = 16, 32, 48: at 400, 500 and 550 rows (32 heads: 5.1 against 5.6 us at 64,
+// 6.6 against 6.2 at 640, 14.3 against 9.4 at 4,096).  Few heads make the sums' LDS chain of 256 / H rows long, many
+// spread the direct form over the chip: H = 2 crosses at 1,200 rows, 128 at 2,700, 300 at 4,096.
+int64_t gate_direct_rows(int64_t H) { return H < 8 ? 2048 : H <= 64 ? 512 : 4096; }
+
+// The groups of rows that gates_bwd_sums_kernel's workgroups take, `per` rows each: one pass of rows a workgroup (an
+// element a lane) up to 512 groups, then as many passes as keep to that (the second stage adds the groups' sums).
 int64_t gate_groups(int64_t rows, int64_t H, int64_t* per) {
   const int64_t rpp = H < GATE_THREADS ? GATE_THREADS / H : 1;
   *per = rpp * ((rows + rpp * 512 - 1) / (rpp * 512));
@@ -703,8 +723,13 @@ int macai_gdr_gates_fwd_typed(const void* b, const void* a, const void* A_log, i
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)((n + GATE_THREADS - 1) / GATE_THREADS));
   const GateParams gp{A_log, dt_bias, atype, dtype_bias};
-  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_fwd_kernel<PT>), grid, dim3(GATE_THREADS), 0, st, (const PT*)b,
-                                        (const PT*)a, gp, params, beta, g, n, (int)H))
+  if (atype != MACAI_GDR_F32 || dtype_bias != MACAI_GDR_F32 || params) {
+    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_fwd_kernel<PT, true>), grid, dim3(GATE_THREADS), 0, st, (const PT*)b,
+                                          (const PT*)a, gp, params, beta, g, n, (int)H))
+  } else {
+    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_fwd_kernel<PT, false>), grid, dim3(GATE_THREADS), 0, st, (const PT*)b,
+                                          (const PT*)a, gp, params, beta, g, n, (int)H))
+  }
   return launched(what);
 }
 
@@ -720,9 +745,9 @@ int64_t macai_gdr_gates_partials(int64_t n, int64_t H) {
   return gate_groups(n / H, H, &per) * 2 * H;
 }
 
-static int gates_bwd(const char* what, const void* b, const void* a, const float* A_log, const float* dt_bias,
-                     const float* dbeta, const float* dg, void* db, void* da, double* part, int64_t n, int64_t H,
-                     int32_t dtype, void* stream) {
+static int check_gates_bwd(const char* what, const void* b, const void* a, const float* A_log, const float* dt_bias,
+                           const float* dbeta, const float* dg, void* db, void* da, int64_t n, int64_t H,
+                           int32_t dtype) {
   if (n < 1 || H < 1 || n % H) return fail(MACAI_GDR_EINVAL, "%s: need n >= 1 a multiple of H >= 1", what);
   if (dtype < MACAI_GDR_F32 || dtype > MACAI_GDR_F16) return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
   if (!b || !a || !A_log || !dt_bias || !dbeta || !dg || !db || !da)
@@ -730,17 +755,21 @@ static int gates_bwd(const char* what, const void* b, const void* a, const float
   const void* ps[] = {b, a, dbeta, dg, db, da};
   for (const void* p : ps)
     if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
-  int64_t per;
-  const int64_t rows = n / H, groups = gate_groups(rows, H, &per);
-  hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)groups), block(GATE_THREADS);
-  if (part) {
-    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_kernel<PT, true>), grid, block, 0, st, (const PT*)b, (const PT*)a,
-                                          A_log, dt_bias, dbeta, dg, (PT*)db, (PT*)da, part, rows, (int)H, (int)per))
-  } else {
-    DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_kernel<PT, false>), grid, block, 0, st, (const PT*)b, (const PT*)a,
-                                          A_log, dt_bias, dbeta, dg, (PT*)db, (PT*)da, part, rows, (int)H, (int)per))
-  }
+  return MACAI_GDR_OK;
+}
+
+// gates_bwd_kernel and, with dA_log non-null, gates_params_direct_kernel.
+static int gates_bwd_direct(const char* what, const void* b, const void* a, const float* A_log, const float* dt_bias,
+                            const float* dbeta, const float* dg, void* db, void* da, void* dA_log, int32_t atype,
+                            void* ddt_bias, int32_t dtype_bias, int64_t n, int64_t H, int32_t dtype, hipStream_t st) {
+  const dim3 grid((unsigned)((n + GATE_THREADS - 1) / GATE_THREADS));
+  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_kernel<PT>), grid, dim3(GATE_THREADS), 0, st, (const PT*)b,
+                                        (const PT*)a, A_log, dt_bias, dbeta, dg, (PT*)db, (PT*)da, n, (int)H))
+  if (int rc = launched(what)) return rc;
+  if (!dA_log) return MACAI_GDR_OK;
+  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_params_direct_kernel<PT>), dim3((unsigned)H), dim3(256), 0, st,
+                                        (const PT*)a, A_log, dt_bias, dg, dA_log, ddt_bias, atype, dtype_bias, n / H,
+                                        (int)H))
   return launched(what);
 }
 
@@ -749,12 +778,9 @@ int macai_gdr_gates_bwd(const void* b, const void* a, const float* A_log, const 
                         int32_t dtype, void* stream) {
   const char* what = "macai_gdr_gates_bwd";
   if (!dA_log != !ddt_bias) return fail(MACAI_GDR_EINVAL, "%s: dA_log and ddt_bias go together", what);
-  if (int rc = gates_bwd(what, b, a, A_log, dt_bias, dbeta, dg, db, da, nullptr, n, H, dtype, stream)) return rc;
-  if (!dA_log) return MACAI_GDR_OK;
-  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_params_direct_kernel<PT>), dim3((unsigned)H), dim3(256), 0,
-                                        (hipStream_t)stream, (const PT*)a, A_log, dt_bias, dg, dA_log, ddt_bias, n / H,
-                                        (int)H))
-  return launched(what);
+  if (int rc = check_gates_bwd(what, b, a, A_log, dt_bias, dbeta, dg, db, da, n, H, dtype)) return rc;
+  return gates_bwd_direct(what, b, a, A_log, dt_bias, dbeta, dg, db, da, dA_log, MACAI_GDR_F32, ddt_bias, MACAI_GDR_F32,
+                          n, H, dtype, (hipStream_t)stream);
 }
 
 int macai_gdr_gates_bwd_typed(const void* b, const void* a, const float* A_log, const float* dt_bias,
@@ -765,11 +791,20 @@ int macai_gdr_gates_bwd_typed(const void* b, const void* a, const float* A_log, 
   if (!part || !dA_log || !ddt_bias) return fail(MACAI_GDR_EINVAL, "%s: null pointer", what);
   if (!param_type_ok(atype) || !param_type_ok(dtype_bias)) return fail(MACAI_GDR_EUNSUP, "%s: dtype code", what);
   if (((uintptr_t)part & 7u) != 0) return fail(MACAI_GDR_EINVAL, "%s: the partial sums must be 8-byte aligned", what);
-  if (int rc = gates_bwd(what, b, a, A_log, dt_bias, dbeta, dg, db, da, part, n, H, dtype, stream)) return rc;
+  if (int rc = check_gates_bwd(what, b, a, A_log, dt_bias, dbeta, dg, db, da, n, H, dtype)) return rc;
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t rows = n / H;
+  if (rows <= gate_direct_rows(H))
+    return gates_bwd_direct(what, b, a, A_log, dt_bias, dbeta, dg, db, da, dA_log, atype, ddt_bias, dtype_bias, n, H,
+                            dtype, st);
   int64_t per;
-  const int64_t groups = gate_groups(n / H, H, &per);
-  hipLaunchKernelGGL(gates_params_kernel, dim3((unsigned)H), dim3(64), 0, (hipStream_t)stream, part, dA_log, ddt_bias,
-                     atype, dtype_bias, (int)groups, (int)H);
+  const int64_t groups = gate_groups(rows, H, &per), hblocks = (H + GATE_THREADS - 1) / GATE_THREADS;
+  DISPATCH_PT(dtype, hipLaunchKernelGGL((gates_bwd_sums_kernel<PT>), dim3((unsigned)(groups * hblocks)),
+                                        dim3(GATE_THREADS), 0, st, (const PT*)b, (const PT*)a, A_log, dt_bias, dbeta, dg,
+                                        (PT*)db, (PT*)da, part, rows, (int)H, (int)per, (int)hblocks))
+  if (int rc = launched(what)) return rc;
+  hipLaunchKernelGGL(gates_params_kernel, dim3((unsigned)H), dim3(64), 0, st, part, dA_log, ddt_bias, atype, dtype_bias,
+                     (int)groups, (int)H);
   return launched(what);
 }
 

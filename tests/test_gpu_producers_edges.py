@@ -7,6 +7,7 @@ plus 2^-20 of the 2-norm (eight such roundings of terms that cancel by half)."""
 import pytest
 import torch
 
+from macai.gated_delta import _native as N
 from macai.layer import conv_qkv, gates
 from oracle import producers as P
 from oracle.gdr import rel
@@ -55,6 +56,34 @@ def test_gates_rows_and_heads(rows, H, dtype, ptypes):
     xs = [_draw((rows, H), dtype, gen), _draw((rows, H), dtype, gen, 3.0), _draw((H,), ptypes[0], gen),
           _draw((H,), ptypes[1], gen)]
     _compare(gates, P.gates, xs, gen)
+
+
+@pytest.mark.parametrize("ptypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.float16)])
+@pytest.mark.parametrize("rows,H", [(512, 16), (513, 16), (513, 64), (2048, 3), (2049, 3), (4096, 65), (4097, 65),
+                                    (4097, 257), (2600, 8)])
+def test_gates_parameter_gradients_on_both_forms(rows, H, ptypes):
+    """Both sides of the line between the two forms of A_log's and dt_bias's gradients, and more heads than a
+    workgroup's lanes past it: the float64 oracle's; and the entry point without scratch, which always takes the pass of
+    a workgroup a head: the same db and da bit for bit, its float32 sums within two roundings of the others'."""
+    print("case gates parameters", rows, H, ptypes, flush=True)
+    gen = torch.Generator().manual_seed(rows + H)
+    xs = [_draw((rows, H), torch.bfloat16, gen), _draw((rows, H), torch.bfloat16, gen, 3.0), _draw((H,), ptypes[0], gen),
+          _draw((H,), ptypes[1], gen)]
+    _compare(gates, P.gates, xs, gen)
+    b, a, rate, bias = (x.cuda() for x in xs)
+    rate, bias = rate.float(), bias.float()
+    db_up, dg_up = (_draw((rows, H), torch.float32, gen).cuda() for _ in range(2))
+    f32 = lambda: torch.empty(H, device="cuda")
+    n, code, p, st = rows * H, N.BF16, N.ptr, N.stream_of(b)
+    part = torch.empty(N.lib().macai_gdr_gates_partials(n, H), dtype=torch.float64, device="cuda")
+    got = [[torch.empty_like(b), torch.empty_like(a), f32(), f32()] for _ in range(2)]
+    ins = [p(x) for x in (b, a, rate, bias, db_up, dg_up)]
+    N.call("macai_gdr_gates_bwd", *ins, *(p(x) for x in got[0]), n, H, code, st)
+    d_b, d_a, d_rate, d_bias = (p(x) for x in got[1])
+    N.call("macai_gdr_gates_bwd_typed", *ins, d_b, d_a, p(part), d_rate, N.F32, d_bias, N.F32, n, H, code, st)
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    for x, y in zip(got[0][2:], got[1][2:]):   # double sums in two orders: past their roundings to float32 2^-52 a term
+        assert rel(x.double().cpu(), y.double().cpu()) < 2.0 ** -23
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
