@@ -3872,10 +3872,12 @@ int macai_gdr_state_scan(const float* maps, const float* s0, float* starts, int6
 // form (DK = DV, more chunk-heads than CUs) with two value heads a key head, where a workgroup can run both of a key
 // head's in turn without a longer run: 2 ceil(units / 2 / CUs) chunk-heads the longest instead of ceil(units / CUs).
 // (One more chunk-head a run costs about 20 us at 128 x 128.  Folding saves the two group_sum launches and the per-head
-// rows they read: a training step of 1,024 chunk-heads 254 -> 244 us, of 8,192 1,824 -> 1,771.)
+// rows they read: a training step of 1,024 chunk-heads 254 -> 244 us, of 8,192 1,824 -> 1,771.)  The widths are the
+// bf16 kernels' (check_common).
 static bool cb8_folds(int64_t units, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int dtype, int64_t cus) {
-  return dtype == MACAI_GDR_BF16 && DK == DV && Hk > 0 && H == 2 * Hk && cus > 0 && units > cus &&
-         units < (int64_t)1 << 30 && 2 * ((units / 2 + cus - 1) / cus) <= (units + cus - 1) / cus;
+  return dtype == MACAI_GDR_BF16 && DK == DV && (DK == 32 || DK == 64 || DK == 128) && Hk > 0 && H == 2 * Hk &&
+         cus > 0 && units > cus && units < (int64_t)1 << 30 &&
+         2 * ((units / 2 + cus - 1) / cus) <= (units + cus - 1) / cus;
 }
 
 int macai_gdr_chunk_bwd_folds(int64_t B, int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype,

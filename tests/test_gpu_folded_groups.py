@@ -47,3 +47,9 @@ def test_folding_rule():
         1, 64 * chunks, H, Hk, D, DV, dtype, None, 0)
     assert [folds(n) for n in (16, 20, 32, 39, 64)] == [0, 1, 1, 0, 1]
     assert not folds(64, DV=64) and not folds(64, Hk=16) and not folds(64, Hk=4) and not folds(64, dtype=N.F32)
+
+
+def test_folds_only_the_widths_the_kernel_takes():
+    """At widths that the bf16 per-chunk backward does not take, the rule says no, as the folded entry point does."""
+    folds = lambda D: N.lib().macai_gdr_chunk_bwd_folds(1, 64 * 64, 16, 8, D, D, N.BF16, None, 0)
+    assert [D for D in range(32, 257, 32) if folds(D)] == [32, 64, 128]
