@@ -618,10 +618,11 @@ def plan(B: int, T: int, H: int, DK: int, DV: int, save: bool, Hk: int = None, d
     """What a drop-in call of these dimensions runs under the current settings (the reference's plan, op.py:105-113,
     for this build's kernels): the chunk length (64 for every pass), the operand type, the forward's segments, value
     split and state-pass kernel, and -- when the forward saves for a backward -- whether the backward recomputes
-    (RECOMPUTE_STATES) and reruns prep (KEEP_PREP), its state passes, their split, the per-chunk backward's kernel and
-    the operands of a backward that receives a gradient of the final state (BF16_STATE_GRAD).  cus: the device's
-    compute units (the persistent per-chunk backward runs where there are more chunk-heads than CUs); l2norm: the call's
-    use_qk_l2norm_in_kernel."""
+    (RECOMPUTE_STATES) and reruns prep (KEEP_PREP), its state passes, their split, the per-chunk backward's kernel, what
+    sums a key head's dq and dk over its value heads (head_sum: None without grouped heads, "chunk_bwd" where the
+    per-chunk backward does, "group_sum" where two launches after it do) and the operands of a backward that receives a
+    gradient of the final state (BF16_STATE_GRAD).  cus: the device's compute units (the persistent per-chunk backward
+    runs where there are more chunk-heads than CUs); l2norm: the call's use_qk_l2norm_in_kernel."""
     Hk = Hk or H
     cdt = compute_dtype(dtype, DK, DV, save, l2norm and FUSED_NORM, T)
     bf = cdt == torch.bfloat16
@@ -647,6 +648,9 @@ def plan(B: int, T: int, H: int, DK: int, DV: int, save: bool, Hk: int = None, d
         out["bwd_split"] = split_for(B * H, T, DV, 2 if pair else 1)
         units = B * H * NT
         out["chunk_bwd"] = (("chunk_bwd8xn" if DK == DV and units > cus else "chunk_bwd8") if bf else "chunk_bwd")
+        # macai_gdr_chunk_bwd_folds' rule: whole pairs, no workgroup's run longer
+        folds = out["chunk_bwd"] == "chunk_bwd8xn" and H == 2 * Hk and 2 * -(-units // (2 * cus)) <= -(-units // cus)
+        out["head_sum"] = None if Hk == H else "chunk_bwd" if folds else "group_sum"
         # a backward that receives a gradient of the final state (BF16_STATE_GRAD)
         out["state_grad_operands"] = "f32" if bf and not BF16_STATE_GRAD else out["operands"]
     return out

@@ -53,3 +53,13 @@ def test_folds_only_the_widths_the_kernel_takes():
     """At widths that the bf16 per-chunk backward does not take, the rule says no, as the folded entry point does."""
     folds = lambda D: N.lib().macai_gdr_chunk_bwd_folds(1, 64 * 64, 16, 8, D, D, N.BF16, None, 0)
     assert [D for D in range(32, 257, 32) if folds(D)] == [32, 64, 128]
+
+
+def test_plan_reports_the_folding():
+    """op.plan says what macai_gdr_chunk_bwd_folds answers, over chunk counts, widths and groups."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for H, Hk, D in ((16, 8, 128), (2, 1, 64), (32, 16, 32), (8, 2, 128)):
+        for chunks in (1, 16, 17, 20, 32, 39, 64, 129, 300, 1000):
+            folds = N.lib().macai_gdr_chunk_bwd_folds(1, 64 * chunks, H, Hk, D, D, N.BF16, None, 0)
+            p = op.plan(1, 64 * chunks, H, D, D, True, Hk=Hk, cus=cus)
+            assert p["head_sum"] == ("chunk_bwd" if folds else "group_sum"), (H, Hk, D, chunks)

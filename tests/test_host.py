@@ -378,6 +378,17 @@ def test_plan_reports_the_launch_choices():
     assert op.plan(4, 1024, 16, 128, 128, save=True, l2norm=False)["mixed_io"]
     assert not op.plan(4, 1024, 16, 128, 128, save=True, l2norm=False, Hk=4)["mixed_io"]
     assert not op.plan(4, 1024, 16, 128, 128, save=True)["mixed_io"]                     # bf16 operands
+
+
+def test_plan_reports_what_sums_grouped_heads():
+    """Two value heads a key head: the per-chunk backward at 1,024 chunk-heads of 256 compute units, the two launches
+    after it at 624 (a workgroup's run would grow) and up to 256; four value heads a key head and float32 operands
+    always the launches; nothing without groups, nor in a forward that saves nothing."""
+    what = lambda T, H=16, Hk=8, D=128, **kw: op.plan(1, T, H, D, D, save=True, Hk=Hk, **kw)["head_sum"]
+    assert [what(64 * n) for n in (16, 20, 39, 64)] == ["group_sum", "chunk_bwd", "group_sum", "chunk_bwd"]
+    assert what(4096, Hk=4) == what(4096, dtype=torch.float32) == what(4096, D=96) == "group_sum"
+    assert what(4096, D=64) == "chunk_bwd" and what(4096, Hk=16) is None
+    assert "head_sum" not in op.plan(1, 4096, 16, 128, 128, save=False, Hk=8)
     assert not op.plan(4, 1024, 16, 128, 128, save=True, dtype=torch.float32)["mixed_io"]
 
 
