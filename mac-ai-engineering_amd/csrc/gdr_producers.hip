@@ -7,10 +7,10 @@
 //
 // The convolution is an HBM stream: every input and output byte crosses once (the 3-row halos come again through L2).
 // A lane owns a channel vector over consecutive time steps, all its input rows loaded at once, a wave 64 consecutive
-// vectors: 4 channels over 8 steps in the forward (conv_fwd_kernel), 8 bytes over 16 in the backward (conv_bwd_kernel),
-// which forms du = dy silu'(u) for its steps and the 3 after them in registers, dx from du's
-// windows (one writer an element) and the taps' gradient's sums over its steps; a tile of 64 rows adds its waves' sums
-// in order through LDS, sum_columns_kernel the tiles' partials in tile order: deterministic.
+// vectors: 4 channels over 8 steps in the forward (conv_fwd_kernel), 2 over 16 in the backward (conv_bwd_kernel; over few
+// tiles 2 over 4, conv_bwd_few_kernel), which forms du = dy silu'(u) for its steps and the 3 after them in registers, dx
+// from du's windows (one writer an element) and the taps' gradient's sums over its steps; a tile of 64 rows adds its
+// blocks' sums in order through LDS, sum_columns_kernel the tiles' partials in tile order: deterministic.
 // The gates are one pass each way, an element a lane; over many rows the backward's also forms its workgroups' sums of
 // A_log's and dt_bias's gradients, which a second launch adds in a fixed order, over few a second pass takes a workgroup a
 // head (gate_direct_rows).
@@ -54,11 +54,11 @@ __device__ __forceinline__ void from_words(const unsigned (&wd)[N * sizeof(T) / 
   }
 }
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
-// N floats written as T: N * sizeof(T) bytes (8, 16 or 32) in 16-byte stores and at most one 8-byte store.
+// N floats written as T: N * sizeof(T) bytes (4, 8, 16 or 32) in 16-byte stores and at most one narrower one.
 template <typename T, int N>
 __device__ __forceinline__ void store_as(T* p, const float (&x)[N]) {
   constexpr int NW = N * (int)sizeof(T) / 4;
-  static_assert(NW % 2 == 0, "whole 8-byte pieces");
+  static_assert(NW == 1 || NW % 2 == 0, "one word or whole 8-byte pieces");
   unsigned wd[NW];
   to_words<T, N>(x, wd);
   unsigned* q = reinterpret_cast<unsigned*>(p);
@@ -66,6 +66,7 @@ __device__ __forceinline__ void store_as(T* p, const float (&x)[N]) {
   for (int s = 0; s + 4 <= NW; s += 4)
     *reinterpret_cast<u32x4_t*>(q + s) = u32x4_t{wd[s], wd[s + 1], wd[s + 2], wd[s + 3]};
   if constexpr (NW % 4 == 2) *reinterpret_cast<u32x2_t*>(q + NW - 2) = u32x2_t{wd[NW - 2], wd[NW - 1]};
+  if constexpr (NW == 1) *q = wd[0];
 }
 // N values of T from memory as floats, in one load of N * sizeof(T) bytes.
 template <typename T, int N>
@@ -96,12 +97,12 @@ struct ConvArgs {
   int wt;
 };
 
-// Where a 16-byte channel vector lives among the outputs: q, k (key heads, each written REP times: REP = 1 keeps key
-// heads only) or v.  A vector never straddles a head (head widths are multiples of the vector).
+// Where a lane's channel vector (2 or 4 channels) lives among the outputs: q, k (key heads, each written REP times: REP =
+// 1 keeps key heads only) or v.  A vector never straddles a head (head widths are multiples of 8).
 struct Dest {
   int which;                      // 0 q, 1 k, 2 v
   unsigned pitch;                 // row pitch of the destination (elements)
-  unsigned col;                     // the vector's first column there (copy 0)
+  unsigned col;                   // the vector's first column there (copy 0)
   __device__ Dest(int c, int KD, int DK, int REP, int C) {
     if (c < 2 * KD) {
       which = c < KD ? 0 : 1;
@@ -232,30 +233,47 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
   }
 }
 
-// The backward, like the forward, streams: a lane owns 4 channels (2 of 4-byte x) over S consecutive time steps
-// t0 .. t0 + S - 1 and issues all its loads at once -- x[t0 - 3 .. t0 + S + 2] and the upstream gradient
-// dy[t0 .. t0 + S + 2] (q's and k's copies summed in copy order) -- then walks the rows with everything in registers:
+// du = dy s (1 + u (1 - s)), s = sigmoid(u).
+template <bool EXACT>
+__device__ __forceinline__ float silu_grad(float u, float dy) {
+  const float sg = logistic<EXACT>(u);
+  return dy * (sg * (1.0f + u * (1.0f - sg)));
+}
+
+// A tile's share of the taps' gradient: the blocks' double sums (block, then the tile's channels' taps) added in block
+// order.  `out` is the tile's [C, 4]; o0 the workgroup's first element of it, n the elements there.
+template <int SPAN, int BLOCKS, int THREADS>
+__device__ __forceinline__ void add_blocks(const double (&red)[BLOCKS][SPAN], float* out, int o0, int n) {
+  for (int o = threadIdx.x; o < SPAN && o0 + o < n; o += THREADS) {
+    double sum = red[0][o];
+#pragma unroll
+    for (int w = 1; w < BLOCKS; ++w) sum += red[w][o];
+    out[o0 + o] = (float)sum;
+  }
+}
+
+// The backward, like the forward, streams: a lane owns 2 channels over S consecutive time steps t0 .. t0 + S - 1 and
+// issues all its loads at once -- x[t0 - 3 .. t0 + S + 2] and the upstream gradient dy[t0 .. t0 + S + 2] (q's and k's
+// copies summed in copy order) -- then walks the rows with everything in registers:
 //   du[t] = dy s (1 + u (1 - s)), s = sigmoid(u)   (0 past the end), for its S rows and the 3 after them,
 //   dx[t] = w0 du[t + 3] + w1 du[t + 2] + w2 du[t + 1] + w3 du[t],
 //   part[tile][c, j] = sum over the tile's t of du[t] x[t - 3 + j], in double.
 // A workgroup is one tile of 64 rows: 64 / S waves, a time block each, over the same 64 vectors, whose sums meet in
 // LDS in wave order (deterministic).  S + 3 rows of du for S of dx: at S = 16 the recomputed rows cost a fifth of the
-// activations.  4-byte x takes 2 channels a lane, the same bytes: 4 spill at S = 16, and at S = 8 (half as many rows
-// recomputed again) took 92 us against 66 at B = 4, T = 1024, C = 6144 and 142 against 99 at C = 8192 with repeated
-// heads (the LDS form below 80 and 119).  All of a lane's loads are in flight at 2 waves
-// a SIMD.  Its 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27 us at the card's copy rate and its VALU work is about
-// as long.  Measured there: 36 us, 41 with the taps' gradient (its double sums), against 45 and 65 for the form that
-// staged tiles of x and dy in LDS (three barriers, every row through LDS as float32 twice); at C = 8192, T = 2048 82
-// and 97 against 114 and 154.  S = 8 for bf16 was as fast without the taps' gradient and 14 us slower with it; three
-// waves a SIMD spills.
-constexpr int CV_BWD_STEPS = 16;
-template <typename T> constexpr int conv_bwd_vec() { return sizeof(T) == 4 ? 2 : CV_VE; }
+// activations.  Bound by its bytes and its VALU work, about as long: 151 MB at B = 4, T = 1024, C = 6144 in bf16 are 27
+// us at the card's copy rate.  Measured there: 30.8 us, 35.9 with the taps' gradient; at C = 8192 and T = 2048 82 and 91;
+// in float32 54 and 59 at the first size.  Lanes of 4 channels took 33.5 and 43.2, 84 and 107 in bf16 (239 registers, two
+// waves a SIMD, against 124 and four), 8 steps of 2 channels 30.7 and 41.5, 90 and 111, in float32 61 and 68; a form that
+// staged tiles of x and dy in LDS (three barriers, every row through LDS as float32 twice) 40.6 and 60.2, 109 and 160,
+// in float32 63 and 75.
+constexpr int CV_BWD_STEPS = 16, CV_BWD_VE = 2;
 template <typename T, typename TV, bool TAPS>
 __global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_kernel(ConvArgs a) {
-  constexpr int VE = conv_bwd_vec<T>(), S = CV_BWD_STEPS, NWAVE = CV_ROWS / S;
+  constexpr int VE = CV_BWD_VE, S = CV_BWD_STEPS, BLOCKS = CV_ROWS / S;
   constexpr bool EXACT = sizeof(T) == 4;
   constexpr int XR = S + 2 * CV_HALO, DR = S + CV_HALO;
-  __shared__ double red[TAPS ? NWAVE : 1][TAPS ? VE : 1][64];   // one tap's sums: a row a wave
+  constexpr int SPAN = CV_TAPS * VE * 64;      // the taps' gradients of the tile's channels
+  __shared__ __attribute__((aligned(16))) double red[TAPS ? BLOCKS : 1][TAPS ? SPAN : 1];   // a wave's sums a row
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int cl = (blockIdx.x * 64 + lane) * VE;
   const bool on = cl < a.C;                // lanes past the channels repeat the last vector and store nothing
@@ -264,11 +282,11 @@ __global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_ker
   const int row0 = b * Tn;                 // B T C < 2^31
   typedef unsigned wordx_t __attribute__((ext_vector_type(VE * sizeof(T) / 4)));
   typedef unsigned wordv_t __attribute__((ext_vector_type(VE * sizeof(TV) / 4)));
-  double acc[CV_TAPS][VE];
+  double acc[VE][CV_TAPS];
 #pragma unroll
-  for (int j = 0; j < CV_TAPS; ++j)
+  for (int i = 0; i < VE; ++i)
 #pragma unroll
-    for (int i = 0; i < VE; ++i) acc[j][i] = 0.0;
+    for (int j = 0; j < CV_TAPS; ++j) acc[i][j] = 0.0;
   if (t0 < Tn) {                           // the waves past the end only join the sums
     // rows outside the sequence read a row inside it, so that every load is unconditional; the waves that have such
     // rows (their first or last block) zero them after
@@ -333,6 +351,7 @@ __global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_ker
     }
 #pragma unroll
     for (int s = 0; s < DR; ++s) {
+      if (t0 + s - CV_HALO >= Tn) break;   // past the end: du is 0 and there is no dx
 #pragma unroll
       for (int j = 0; j + 1 < CV_TAPS; ++j)
 #pragma unroll
@@ -347,17 +366,16 @@ __global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_ker
 #pragma unroll
       for (int i = 0; i < VE; ++i) {
         const float uu = tap_dot<EXACT, VE>(tw, i, xw[0][i], xw[1][i], xw[2][i], xw[3][i]);
-        const float sg = logistic<EXACT>(uu);
-        dw[3][i] = g[s][i] * (sg * (1.0f + uu * (1.0f - sg)));
+        dw[3][i] = silu_grad<EXACT>(uu, g[s][i]);
       }
       if (TAPS && s < S)
 #pragma unroll
         for (int i = 0; i < VE; ++i) {
           const double dd = (double)dw[3][i];
 #pragma unroll
-          for (int j = 0; j < CV_TAPS; ++j) acc[j][i] = fma(dd, (double)xw[j][i], acc[j][i]);
+          for (int j = 0; j < CV_TAPS; ++j) acc[i][j] = fma(dd, (double)xw[j][i], acc[i][j]);
         }
-      if (s >= CV_HALO && on && t0 + s - CV_HALO < Tn) {
+      if (s >= CV_HALO && on) {
         float o[VE];
 #pragma unroll
         for (int i = 0; i < VE; ++i) o[i] = tap_dot<EXACT, VE>(tw, i, dw[3][i], dw[2][i], dw[1][i], dw[0][i]);
@@ -366,22 +384,128 @@ __global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_ker
     }
   }
   if constexpr (TAPS) {
-    // tap by tap: every wave's sums into LDS, then wave w adds channel i = w's over the waves in order
-    float* out = a.part + (size_t)(b * a.ntiles + blockIdx.y) * a.C * CV_TAPS;
+    double* mine = &red[wave][lane * VE * CV_TAPS];
 #pragma unroll
-    for (int j = 0; j < CV_TAPS; ++j) {
-      if (j) __syncthreads();              // the previous tap's sums are read
+    for (int i = 0; i < VE; ++i)
 #pragma unroll
-      for (int i = 0; i < VE; ++i) red[wave][i][lane] = acc[j][i];
-      __syncthreads();
-      if (wave < VE && on) {
-        double s = red[0][wave][lane];
+      for (int j = 0; j < CV_TAPS; ++j) mine[i * CV_TAPS + j] = acc[i][j];
+    __syncthreads();
+    add_blocks<SPAN, BLOCKS, 64 * BLOCKS>(red, a.part + (size_t)(b * a.ntiles + blockIdx.y) * a.C * CV_TAPS,
+                                          blockIdx.x * SPAN, a.C * CV_TAPS);
+  }
+}
+
+// The same over few tiles (conv_few), where the form above leaves compute units idle and a lane's 19 rows in turn are the
+// time: a workgroup is a tile of 64 rows by 16 vectors, a lane 4 steps of one, and the 3 rows of du after a lane's own
+// come through LDS from the lanes that own them (the rows after the tile are formed by its first three blocks of steps).
+// Every element's arithmetic is the form's above: dx has the same bits; the taps' sums group by 4 rows.  Bound by
+// latency: one row of 64 tokens, C = 6144, with the taps' gradient 6.4 us in bf16 and 6.8 in float32, of which the second
+// stage's launch is 2.3, against 8.5 and 10.2 of the form above (the LDS form 9.3 and 7.6).  Tiles 8 or 32 vectors wide
+// and 8 steps a lane are slower over few tiles.
+constexpr int CV_FEW_STEPS = 4, CV_FEW_WIDE = 16;
+template <typename T, typename TV, bool TAPS>
+__global__ void __launch_bounds__(CV_FEW_WIDE * (CV_ROWS / CV_FEW_STEPS)) conv_bwd_few_kernel(ConvArgs a) {
+  constexpr int VE = CV_BWD_VE, S = CV_FEW_STEPS, WIDE = CV_FEW_WIDE, BLOCKS = CV_ROWS / S;
+  constexpr bool EXACT = sizeof(T) == 4;
+  constexpr int XR = S + CV_HALO, SPAN = CV_TAPS * VE * WIDE;
+  static_assert(S > CV_HALO && BLOCKS > CV_HALO, "a block holds the next one's halo, the first blocks the tile's");
+  __shared__ __attribute__((aligned(16))) double red[TAPS ? BLOCKS : 1][TAPS ? SPAN : 1];
+  __shared__ float head[BLOCKS + 1][CV_HALO][WIDE][VE];   // du of each block's first rows; then the rows after the tile
+  const int vec = threadIdx.x % WIDE, block = threadIdx.x / WIDE;
+  const int cl = (blockIdx.x * WIDE + vec) * VE;
+  const bool on = cl < a.C;                // lanes past the channels repeat the last vector and store nothing
+  const int c = on ? cl : a.C - VE;
+  const int b = blockIdx.z, Tn = a.T, end = (blockIdx.y + 1) * CV_ROWS, t0 = blockIdx.y * CV_ROWS + block * S;
+  const int row0 = b * Tn;                 // B T C < 2^31
+  auto row_of = [&](int t) { return (size_t)(unsigned)(row0 + (t < 0 ? 0 : t < Tn ? t : Tn - 1)); };
+  const Dest d(c, a.KD, a.DK, a.REP, a.C);
+  // x[t0 - 3 + i], dy[t0 + i] and the row after the tile that the first blocks form, du[end + block]; loads are of rows
+  // inside the sequence, masked after
+  float xr[XR][VE], g[S][VE], ex[CV_TAPS][VE], eg[VE];
+  const bool extra = block < CV_HALO;
+  auto load_x = [&](int t, float (&r)[VE]) { load_as<T, VE>((const T*)a.x + row_of(t) * a.C + c, r); };
+  auto mask = [&](int t, float (&r)[VE]) {
 #pragma unroll
-        for (int w = 1; w < NWAVE; ++w) s += red[w][wave][lane];
-        out[(size_t)(c + wave) * CV_TAPS + j] = (float)s;
+    for (int i = 0; i < VE; ++i) r[i] = t >= 0 && t < Tn ? r[i] : 0.f;
+  };
+  float du[S + CV_HALO][VE], tw[CV_TAPS][VE];
+#pragma unroll
+  for (int i = 0; i < XR; ++i) load_x(t0 - CV_HALO + i, xr[i]);
+  if (extra)
+#pragma unroll
+    for (int j = 0; j < CV_TAPS; ++j) load_x(end + block - CV_HALO + j, ex[j]);
+  if (d.which == 2) {
+    const TV* src = (const TV*)a.dv + d.col;
+#pragma unroll
+    for (int i = 0; i < S; ++i) load_as<TV, VE>(src + row_of(t0 + i) * d.pitch, g[i]);
+    if (extra) load_as<TV, VE>(src + row_of(end + block) * d.pitch, eg);
+  } else {
+    const T* src = (const T*)(d.which == 0 ? a.dq : a.dk) + d.col;
+#pragma unroll
+    for (int i = 0; i < S; ++i) load_as<T, VE>(src + row_of(t0 + i) * d.pitch, g[i]);
+    if (extra) load_as<T, VE>(src + row_of(end + block) * d.pitch, eg);
+    for (int rep = 1; rep < a.REP; ++rep) {   // a repeated key head's copies, added in copy order
+      float h[S][VE], eh[VE];
+      src += a.DK;
+#pragma unroll
+      for (int i = 0; i < S; ++i) load_as<T, VE>(src + row_of(t0 + i) * d.pitch, h[i]);
+      if (extra) load_as<T, VE>(src + row_of(end + block) * d.pitch, eh);
+#pragma unroll
+      for (int e = 0; e < VE; ++e) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) g[i][e] += h[i][e];
+        if (extra) eg[e] += eh[e];
       }
     }
   }
+  tile_taps<VE>(a.w, a.wt, c, tw);
+#pragma unroll
+  for (int i = 0; i < XR; ++i) mask(t0 - CV_HALO + i, xr[i]);
+#pragma unroll
+  for (int i = 0; i < S; ++i) mask(t0 + i, g[i]);
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int i = 0; i < VE; ++i) {
+      du[s][i] = silu_grad<EXACT>(tap_dot<EXACT, VE>(tw, i, xr[s][i], xr[s + 1][i], xr[s + 2][i], xr[s + 3][i]), g[s][i]);
+      if (s < CV_HALO) head[block][s][vec][i] = du[s][i];
+    }
+  if (extra) {
+#pragma unroll
+    for (int j = 0; j < CV_TAPS; ++j) mask(end + block - CV_HALO + j, ex[j]);
+    mask(end + block, eg);
+#pragma unroll
+    for (int i = 0; i < VE; ++i)
+      head[BLOCKS][block][vec][i] = silu_grad<EXACT>(tap_dot<EXACT, VE>(tw, i, ex[0][i], ex[1][i], ex[2][i], ex[3][i]), eg[i]);
+  }
+  if constexpr (TAPS) {
+#pragma unroll
+    for (int i = 0; i < VE; ++i)
+#pragma unroll
+      for (int j = 0; j < CV_TAPS; ++j) {
+        double sum = 0.0;
+#pragma unroll
+        for (int s = 0; s < S; ++s) sum = fma((double)du[s][i], (double)xr[s + j][i], sum);
+        red[block][(vec * VE + i) * CV_TAPS + j] = sum;
+      }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < CV_HALO; ++s)
+#pragma unroll
+    for (int i = 0; i < VE; ++i) du[S + s][i] = head[block + 1][s][vec][i];
+  T* dxb = (T*)a.dx + (size_t)row0 * a.C + c;
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+    if (on && t0 + s < Tn) {
+      float o[VE];
+#pragma unroll
+      for (int i = 0; i < VE; ++i) o[i] = tap_dot<EXACT, VE>(tw, i, du[s + 3][i], du[s + 2][i], du[s + 1][i], du[s][i]);
+      store_as<T, VE>(dxb + (size_t)(t0 + s) * a.C, o);
+    }
+  if constexpr (TAPS)
+    add_blocks<SPAN, BLOCKS, WIDE * BLOCKS>(red, a.part + (size_t)(b * a.ntiles + blockIdx.y) * a.C * CV_TAPS,
+                                            blockIdx.x * SPAN, a.C * CV_TAPS);
 }
 
 // x at element i of an array in the type of code t (uniform), and back.
@@ -621,6 +745,17 @@ int64_t gate_groups(int64_t rows, int64_t H, int64_t* per) {
 
 int64_t conv_tiles(int64_t T) { return (T + CV_ROWS - 1) / CV_ROWS; }
 
+// Up to this many workgroups of conv_bwd_kernel the backward takes conv_bwd_few_kernel.  Where the two cross, without and
+// with the taps' gradient, at 64 rows or more: in bf16 7.3 against 8.1 us and 11.1 against 11.8 at 384 workgroups, 9.6
+// against 8.3 and 14.2 against 11.9 at 512; in float32 (more arithmetic a byte: the recomputed rows weigh more) 20.0
+// against 22.0 and 24.7 against 25.4 at 1,024, 35.0 against 36.0 and 39 against 40 at 2,048, 71 against 54 and 75 against
+// 59 at 3,072.  Rows shorter than a tile leave its lanes idle in the one form and only waves that exit at once in the
+// other: in float32 at T = 16 5.0 against 7.0 at 128 workgroups, 10.0 against 8.1 at 512; at T = 1 about even up to 128.
+int64_t conv_few(int64_t T, int32_t dtype) {
+  if (dtype != MACAI_GDR_F32) return 384;
+  return 256 * (T >= CV_ROWS ? CV_ROWS / CV_BWD_STEPS : (T + CV_BWD_STEPS - 1) / CV_BWD_STEPS);
+}
+
 }  // namespace
 
 #define DISPATCH_PT(code, ...)                                             \
@@ -686,15 +821,22 @@ int macai_gdr_conv_bwd_typed(const void* x, const float* w, const void* dq, cons
   ConvArgs a{x, w, nullptr, nullptr, nullptr, nullptr, dq, dk, dv, dx, dwp, (int)B, (int)T, (int)C, (int)KD, (int)DK,
              (int)REP, ntiles, MACAI_GDR_F32};
   hipStream_t st = (hipStream_t)stream;
-  // 64 vectors of conv_bwd_vec channels by a tile of CV_ROWS steps; a wave a block of CV_BWD_STEPS of them
-  const int64_t span = 64 * (dtype == MACAI_GDR_F32 ? conv_bwd_vec<float>() : conv_bwd_vec<bf16>());
+  const int64_t wide = 64 * CV_BWD_VE;     // channels a workgroup of the streaming form takes
+  const bool few = (C + wide - 1) / wide * ntiles * B <= conv_few(T, dtype);
+  const int64_t span = few ? CV_FEW_WIDE * CV_BWD_VE : wide;
   const dim3 grid((unsigned)((C + span - 1) / span), (unsigned)ntiles, (unsigned)B);
-  const dim3 block(64 * (CV_ROWS / CV_BWD_STEPS));
+  const dim3 threads(few ? CV_FEW_WIDE * (CV_ROWS / CV_FEW_STEPS) : 64 * (CV_ROWS / CV_BWD_STEPS));
+#define CONV_BWD(TAPS)                                                                          \
+  DISPATCH_PT(dtype, DISPATCH_PV(vdtype, {                                                      \
+    if (few) hipLaunchKernelGGL((conv_bwd_few_kernel<PT, PV, TAPS>), grid, threads, 0, st, a);  \
+    else hipLaunchKernelGGL((conv_bwd_kernel<PT, PV, TAPS>), grid, threads, 0, st, a);          \
+  }))
   if (dwp) {
-    DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_kernel<PT, PV, true>), grid, block, 0, st, a)))
+    CONV_BWD(true)
   } else {
-    DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_bwd_kernel<PT, PV, false>), grid, block, 0, st, a)))
+    CONV_BWD(false)
   }
+#undef CONV_BWD
   if (int rc = launched(what)) return rc;
   if (dw) {
     const int n = (int)(C * CV_TAPS);

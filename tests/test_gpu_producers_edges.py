@@ -46,6 +46,27 @@ def test_conv_blocks_and_channels(T, dtype, wdtype):
                  lambda a, b: P.conv_qkv(a, b, kd, dk, rep, dv, repeat), [x, w], gen)
 
 
+@pytest.mark.parametrize("dtype,v_dtype", [(torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32),
+                                           (torch.float16, torch.bfloat16), (torch.float32, torch.bfloat16),
+                                           (torch.float32, torch.float32)])
+@pytest.mark.parametrize("T", [1, 17, 61, 64, 130])
+def test_conv_backward_on_both_forms(T, dtype, v_dtype):
+    """The backward over many tiles (past 1,024 workgroups, every type's line) against the float64 oracle, and its first
+    two rows by themselves, over few: the same dx bit for bit."""
+    print("case conv forms", T, dtype, v_dtype, flush=True)
+    gen = torch.Generator().manual_seed(T)
+    kd, dk, rep, dv, repeat = 8, 8, 2, 8, True
+    x, w = _draw((1030, T, 32), dtype, gen), _draw((32, 1, 4), torch.float32, gen, 0.3)
+    fused = lambda a, b: conv_qkv(a, b, kd, dk, rep, dv, repeat, v_dtype)
+    _compare(fused, lambda a, b: P.conv_qkv(a, b, kd, dk, rep, dv, repeat), [x, w], gen)
+    ups = [_draw(o.shape, o.dtype, gen).cuda() for o in fused(x.cuda(), w.cuda())]
+    dx = []
+    for n in (len(x), 2):
+        leaf, weight = x[:n].cuda().requires_grad_(True), w.cuda().requires_grad_(True)
+        dx.append(torch.autograd.grad(fused(leaf, weight), [leaf, weight], [u[:n].contiguous() for u in ups])[0])
+    assert torch.equal(dx[0][:2], dx[1])
+
+
 @pytest.mark.parametrize("dtype,ptypes", [(torch.bfloat16, (torch.bfloat16, torch.bfloat16)),
                                           (torch.float32, (torch.float32, torch.float32)),
                                           (torch.bfloat16, (torch.float32, torch.float16))])
