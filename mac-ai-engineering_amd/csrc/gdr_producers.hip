@@ -87,14 +87,13 @@ constexpr int CV_HALO = CV_TAPS - 1;
 
 struct ConvArgs {
   const void* x;                  // [B, T, C] in T
-  const void* w;                  // [C, 4] taps, dtype code wt
+  const void* w;                  // [C, 4] taps: the forward's in TW, the backward's float32
   float* taps;                    // forward: the taps' float32 copy for the backward, or null
   void *q, *k, *v;                // forward outputs: q, k [B, T, KD * REP] in T, v [B, T, C - 2 KD] in TV
   const void *dq, *dk, *dv;       // backward inputs, same layouts
   void* dx;                       // [B, T, C] in T
   float* part;                    // [B * ntiles, C * 4] per-tile taps' gradient, or null
   int B, T, C, KD, DK, REP, ntiles;
-  int wt;
 };
 
 // Where a lane's channel vector (2 or 4 channels) lives among the outputs: q, k (key heads, each written REP times: REP =
@@ -117,16 +116,13 @@ struct Dest {
   }
 };
 
-// The tile's taps, tap-major: tw[j][i] = w[c + i, j] for the lane's N channels; w in the type of code wt (uniform).
-template <int N>
-__device__ __forceinline__ void tile_taps(const void* w, int wt, int c, float (&tw)[CV_TAPS][N]) {
+// The lane's taps, tap-major: tw[j][i] = w[c + i, j] for its N channels, w in TW.
+template <typename TW, int N>
+__device__ __forceinline__ void tile_taps(const void* w, int c, float (&tw)[CV_TAPS][N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     float r[CV_TAPS];
-    const size_t at = (size_t)(c + i) * CV_TAPS;
-    if (wt == MACAI_GDR_F32) load_as<float, CV_TAPS>((const float*)w + at, r);
-    else if (wt == MACAI_GDR_BF16) load_as<bf16, CV_TAPS>((const bf16*)w + at, r);
-    else load_as<f16, CV_TAPS>((const f16*)w + at, r);
+    load_as<TW, CV_TAPS>((const TW*)w + (size_t)(c + i) * CV_TAPS, r);
 #pragma unroll
     for (int j = 0; j < CV_TAPS; ++j) tw[j][i] = r[j];
   }
@@ -174,11 +170,13 @@ constexpr int CV_VE = 4;          // channels a lane
 // input rows at once (the 3 halo rows come again through L2), then forms each output from them.  A wave spans 64
 // consecutive vectors of one block of steps (a wave-uniform start: row addresses are scalar and the ends of the row
 // cost the other waves nothing), a workgroup four consecutive blocks.  Bound by its bytes once the chip is full: at
-// B = 4, T = 1024, C = 6144 in bf16 (101 MB, 18 us at the card's copy rate) 23.0 us, at C = 8192 and T = 2048 (268 MB)
-// 49.9 us, 5.4 TB/s.  Lanes of 8 channels (16-byte loads) took 25.0 and 51.5 us (half the waves, twice the registers),
-// 4 or 16 steps 22.9-23.7 and 50.9-52.8; with a correctly rounded division in silu 28.8 and 61 us.
+// B = 4, T = 1024, C = 6144 in bf16 (101 MB, 18 us at the card's copy rate) 19.9 us, at C = 8192 and T = 2048 (268 MB)
+// 43.5 us, 6.2 TB/s.  Lanes of 8 channels (16-byte loads) took 25.0 and 51.5 us (half the waves, twice the registers),
+// 4 or 16 steps 22.9-23.7 and 50.9-52.8; with a correctly rounded division in silu 28.8 and 61 us (of 23.0 and 49.9
+// then).  The taps' type is a template argument: behind branches on its code 2-byte taps were waited for after all of x,
+// 24.1 and 54.1 us (float32 x 39.7 against 34.6, 103 against 96).
 constexpr int CV_FWD_STEPS = 8;
-template <typename T, typename TV>
+template <typename T, typename TV, typename TW>
 __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
   constexpr int VE = CV_VE;
   constexpr bool EXACT = sizeof(T) == 4;
@@ -189,6 +187,8 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
   if (c >= a.C || t0 >= Tn) return;
   typedef unsigned wordx_t __attribute__((ext_vector_type(VE * sizeof(T) / 4)));
   const int row0 = b * Tn;                 // B T C < 2^31
+  float tw[CV_TAPS][VE];                   // the taps first: loads arrive in order, and every output needs them
+  tile_taps<TW, VE>(a.w, c, tw);
   wordx_t xr[NR];                          // x[t0 - 3 + i], zero outside the sequence (see conv_bwd_kernel)
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
@@ -196,8 +196,6 @@ __global__ void __launch_bounds__(256) conv_fwd_kernel(ConvArgs a) {
     const size_t row = (unsigned)(row0 + (t < 0 ? 0 : t < Tn ? t : Tn - 1));
     xr[i] = *reinterpret_cast<const wordx_t*>((const T*)a.x + row * a.C + c);
   }
-  float tw[CV_TAPS][VE];
-  tile_taps<VE>(a.w, a.wt, c, tw);
   if (a.taps && t0 == 0 && b == 0)         // one wave a channel range
 #pragma unroll
     for (int e = 0; e < VE; ++e)
@@ -339,7 +337,7 @@ __global__ void __launch_bounds__(64 * (CV_ROWS / CV_BWD_STEPS), 2) conv_bwd_ker
           for (int e = 0; e < VE; ++e) g[i][e] = 0.f;
     }
     float tw[CV_TAPS][VE];
-    tile_taps<VE>(a.w, a.wt, c, tw);
+    tile_taps<float, VE>(a.w, c, tw);
     T* dxb = (T*)a.dx + (size_t)row0 * a.C + c;
     float xw[CV_TAPS][VE], dw[CV_TAPS][VE];   // x[t - 3 .. t] and du[t - 3 .. t], oldest first
 #pragma unroll
@@ -458,7 +456,7 @@ __global__ void __launch_bounds__(CV_FEW_WIDE * (CV_ROWS / CV_FEW_STEPS)) conv_b
       }
     }
   }
-  tile_taps<VE>(a.w, a.wt, c, tw);
+  tile_taps<float, VE>(a.w, c, tw);
 #pragma unroll
   for (int i = 0; i < XR; ++i) mask(t0 - CV_HALO + i, xr[i]);
 #pragma unroll
@@ -770,6 +768,12 @@ int64_t conv_few(int64_t T, int32_t dtype) {
     case MACAI_GDR_BF16: { using PV = gdr::bf16; __VA_ARGS__; } break;     \
     default: { using PV = gdr::f16; __VA_ARGS__; } break;                  \
   }
+#define DISPATCH_PW(code, ...)                                             \
+  switch (code) {                                                          \
+    case MACAI_GDR_F32: { using PW = float; __VA_ARGS__; } break;          \
+    case MACAI_GDR_BF16: { using PW = gdr::bf16; __VA_ARGS__; } break;     \
+    default: { using PW = gdr::f16; __VA_ARGS__; } break;                  \
+  }
 
 extern "C" {
 
@@ -790,11 +794,12 @@ int macai_gdr_conv_fwd_typed(const void* x, const void* w, int32_t wdtype, float
   for (const void* p : ps)
     if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
   ConvArgs a{x, w, taps, q, k, v, nullptr, nullptr, nullptr, nullptr, nullptr, (int)B, (int)T, (int)C, (int)KD, (int)DK,
-             (int)REP, (int)conv_tiles(T), wdtype};
+             (int)REP, (int)conv_tiles(T)};
   hipStream_t st = (hipStream_t)stream;
   const dim3 grid((unsigned)((C + 64 * CV_VE - 1) / (64 * CV_VE)), (unsigned)((T + 4 * CV_FWD_STEPS - 1) / (4 * CV_FWD_STEPS)),
                   (unsigned)B);
-  DISPATCH_PT(dtype, DISPATCH_PV(vdtype, hipLaunchKernelGGL((conv_fwd_kernel<PT, PV>), grid, dim3(256), 0, st, a)))
+  DISPATCH_PT(dtype, DISPATCH_PV(vdtype, DISPATCH_PW(wdtype, hipLaunchKernelGGL((conv_fwd_kernel<PT, PV, PW>), grid,
+                                                                                dim3(256), 0, st, a))))
   return launched(what);
 }
 
@@ -819,7 +824,7 @@ int macai_gdr_conv_bwd_typed(const void* x, const float* w, const void* dq, cons
     if (!aligned16(p)) return fail(MACAI_GDR_EINVAL, "%s: pointers must be 16-byte aligned", what);
   const int ntiles = (int)conv_tiles(T);
   ConvArgs a{x, w, nullptr, nullptr, nullptr, nullptr, dq, dk, dv, dx, dwp, (int)B, (int)T, (int)C, (int)KD, (int)DK,
-             (int)REP, ntiles, MACAI_GDR_F32};
+             (int)REP, ntiles};
   hipStream_t st = (hipStream_t)stream;
   const int64_t wide = 64 * CV_BWD_VE;     // channels a workgroup of the streaming form takes
   const bool few = (C + wide - 1) / wide * ntiles * B <= conv_few(T, dtype);

@@ -158,3 +158,26 @@ def test_conv_far_negative():
         for o, r in [*zip((o.reshape(T, 8) for o in out), parts), (dx.reshape(T, C), dwant.reshape(T, C))]:
             e = ((o.detach().cpu().double() - r) / r).abs().max().item()
             assert e < 2.0 ** -BITS[o.dtype] + 4 * 89 * 2.0 ** -24, (v_dtype, o.dtype, e)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_untyped_convolution_entry_points(dtype):
+    """macai_gdr_conv_fwd and macai_gdr_conv_bwd take float32 taps: the bits of the typed ones for every output."""
+    print("case conv untyped", dtype, flush=True)
+    gen = torch.Generator().manual_seed(3)
+    B, T, kd, dk, dv = 2, 70, 24, 8, 8
+    C = 2 * kd + 3 * dv
+    p, code = N.ptr, N.dtype_code(dtype)
+    x, w = _draw((B, T, C), dtype, gen).cuda(), _draw((C, 4), torch.float32, gen, 0.3).cuda()
+    ups = [_draw((B, T, 3, d), dtype, gen).cuda() for d in (dk, dk, dv)]
+    sizes = (B, T, C, kd, dk, 1, dv, code, code, N.stream_of(x))
+    nan = lambda *s, d=dtype: torch.full(s, float("nan"), dtype=d, device="cuda")
+    got = []
+    for typed in (False, True):
+        outs = [nan(B, T, 3, d) for d in (dk, dk, dv)] + [nan(B, T, C), nan(C, 4, d=torch.float32)]
+        part = nan(N.lib().macai_gdr_conv_partials(B, T, C), d=torch.float32)
+        to, wt = ("_typed", [N.F32]) if typed else ("", [])
+        N.call("macai_gdr_conv_fwd" + to, p(x), p(w), *wt, *([None] if typed else []), *map(p, outs[:3]), *sizes)
+        N.call("macai_gdr_conv_bwd" + to, p(x), p(w), *map(p, ups), p(outs[3]), p(part), p(outs[4]), *wt, *sizes)
+        got.append(outs)
+    assert all(a.isfinite().all() and torch.equal(a, b) for a, b in zip(*got))
