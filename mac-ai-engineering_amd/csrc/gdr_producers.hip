@@ -728,10 +728,14 @@ int check_conv(const char* what, int64_t B, int64_t T, int64_t C, int64_t KD, in
 
 // Up to this many rows the parameters' gradients come from gates_params_direct_kernel (a workgroup a head), whose
 // chain is then the shorter one; past them from gates_bwd_sums_kernel and gates_params_kernel.  Where the two cross, with
-// the pass over the elements in each, at H = 16, 32, 48: at 400, 500 and 550 rows (32 heads: 5.1 against 5.6 us at 64,
-// 6.6 against 6.2 at 640, 14.3 against 9.4 at 4,096).  Few heads make the sums' LDS chain of 256 / H rows long, many
-// spread the direct form over the chip: H = 2 crosses at 1,200 rows, 128 at 2,700, 300 at 4,096.
-int64_t gate_direct_rows(int64_t H) { return H < 8 ? 2048 : H <= 64 ? 512 : 4096; }
+// the pass over the elements in each: at 8 to 64 heads 500 to 650 rows (16 heads: 5.7 against 6.2 us at 64, 7.6 against 6.4
+// at 1,024, 14.6 against 7.6 at 4,096).  Few heads make the sums' LDS chain of 256 / H rows long: 1 head crosses at 2,050
+// rows, 2 at 1,050, 3 to 7 at 500 to 750.  Many spread the direct form over the chip: 65 cross at 2,050, 96 and 128 at
+// 2,600, 192 and 256 at 2,900 to 3,300, more than 256 between 2,500 and 4,100.
+int64_t gate_direct_rows(int64_t H) {
+  if (H <= 2) return 2048 / H;
+  return H <= 64 ? 576 : H <= 256 ? 2560 : 4096;
+}
 
 // The groups of rows that gates_bwd_sums_kernel's workgroups take, `per` rows each: one pass of rows a workgroup (an
 // element a lane) up to 512 groups, then as many passes as keep to that (the second stage adds the groups' sums).

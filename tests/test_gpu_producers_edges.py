@@ -80,8 +80,8 @@ def test_gates_rows_and_heads(rows, H, dtype, ptypes):
 
 
 @pytest.mark.parametrize("ptypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.float16)])
-@pytest.mark.parametrize("rows,H", [(512, 16), (513, 16), (513, 64), (2048, 3), (2049, 3), (4096, 65), (4097, 65),
-                                    (4097, 257), (2600, 8)])
+@pytest.mark.parametrize("rows,H", [(512, 16), (576, 16), (577, 16), (577, 64), (2048, 1), (2049, 1), (1024, 2), (1025, 2),
+                                    (2048, 3), (2049, 3), (2560, 65), (2561, 65), (4096, 257), (4097, 257), (2600, 8)])
 def test_gates_parameter_gradients_on_both_forms(rows, H, ptypes):
     """Both sides of the line between the two forms of A_log's and dt_bias's gradients, and more heads than a
     workgroup's lanes past it: the float64 oracle's; and the entry point without scratch, which always takes the pass of
