@@ -446,28 +446,35 @@ def bench_producers(cfg, reps=20):
     bf, f32 = torch.bfloat16, torch.float32
     gen = torch.Generator(device=dev).manual_seed(5)
     rnd = lambda *sh, dt=bf: torch.randn(*sh, device=dev, generator=gen).to(dt)
-    x, w4 = rnd(B, T, C), rnd(C, 4, dt=f32) * 0.3
+    x, w4 = rnd(B, T, C), (rnd(C, 4, dt=f32) * 0.3).to(bf)
+    taps = torch.empty(C, 4, device=dev)   # the taps' float32 copy: the forward writes it, the backward reads it
     q, k, v = rnd(B, T, Hk, DK), rnd(B, T, Hk, DK), rnd(B, T, Hv, DV)
     dq, dk, dv, dx = rnd(B, T, Hk, DK), rnd(B, T, Hk, DK), rnd(B, T, Hv, DV), torch.empty(B, T, C, device=dev,
                                                                                           dtype=bf)
     dwp = torch.empty(N.lib().macai_gdr_conv_partials(B, T, C), device=dev, dtype=f32)
-    dw = torch.empty(C, 4, device=dev, dtype=f32)
-    b, a, A_log, dt = rnd(B, T, Hv), rnd(B, T, Hv), torch.zeros(Hv, device=dev), torch.zeros(Hv, device=dev)
-    beta, g, dbeta, dg = (rnd(B, T, Hv, dt=f32) for _ in range(4))
-    db, da, dA, ddt = rnd(B, T, Hv), rnd(B, T, Hv), torch.empty(Hv, device=dev), torch.empty(Hv, device=dev)
-    P, st, BF = N.ptr, N.stream_of(x), N.BF16
+    dw = torch.empty_like(w4)
     n = B * T * Hv
+    b, a, A_log, dt = rnd(B, T, Hv), rnd(B, T, Hv), torch.zeros(Hv, device=dev, dtype=bf), rnd(Hv)
+    params = torch.empty(2, Hv, device=dev)   # A_log's and dt_bias's float32 copies, as the taps'
+    beta, g, dbeta, dg = (rnd(B, T, Hv, dt=f32) for _ in range(4))
+    db, da, dA, ddt = rnd(B, T, Hv), rnd(B, T, Hv), torch.empty_like(A_log), torch.empty_like(dt)
+    part = torch.empty(N.lib().macai_gdr_gates_partials(n, Hv), device=dev, dtype=torch.float64)
+    P, st, BF = N.ptr, N.stream_of(x), N.BF16
+    sizes = (B, T, C, kd, DK, 1, DV, BF, BF, st)
+    gates_in = (P(b), P(a), P(params[0]), P(params[1]), P(dbeta), P(dg), P(db), P(da))
+    # as the layer's training step calls them, its parameters in bf16: each backward with and without their gradients
     calls = {
-        "conv_fwd": (("macai_gdr_conv_fwd", P(x), P(w4), P(q), P(k), P(v), B, T, C, kd, DK, 1, DV, BF, BF, st),
+        "conv_fwd": (("macai_gdr_conv_fwd_typed", P(x), P(w4), BF, P(taps), P(q), P(k), P(v), *sizes),
                      2 * B * T * C * 2),
-        "conv_bwd": (("macai_gdr_conv_bwd", P(x), P(w4), P(dq), P(dk), P(dv), P(dx), None, None, B, T, C, kd, DK, 1,
-                      DV, BF, BF, st), 3 * B * T * C * 2),
-        "conv_bwd_dw": (("macai_gdr_conv_bwd", P(x), P(w4), P(dq), P(dk), P(dv), P(dx), P(dwp), P(dw), B, T, C, kd,
-                         DK, 1, DV, BF, BF, st), 3 * B * T * C * 2 + 2 * dwp.numel() * 4),
-        "gates_fwd": (("macai_gdr_gates_fwd", P(b), P(a), P(A_log), P(dt), P(beta), P(g), n, Hv, BF, st),
-                      n * (2 * 2 + 2 * 4)),
-        "gates_bwd": (("macai_gdr_gates_bwd", P(b), P(a), P(A_log), P(dt), P(dbeta), P(dg), P(db), P(da), None, None,
-                       n, Hv, BF, st), n * (2 * 2 + 2 * 4 + 2 * 2)),
+        "conv_bwd": (("macai_gdr_conv_bwd_typed", P(x), P(taps), P(dq), P(dk), P(dv), P(dx), None, None, BF, *sizes),
+                     3 * B * T * C * 2),
+        "conv_bwd_dw": (("macai_gdr_conv_bwd_typed", P(x), P(taps), P(dq), P(dk), P(dv), P(dx), P(dwp), P(dw), BF,
+                         *sizes), 3 * B * T * C * 2 + 2 * dwp.numel() * 4),
+        "gates_fwd": (("macai_gdr_gates_fwd_typed", P(b), P(a), P(A_log), BF, P(dt), BF, P(params), P(beta), P(g), n,
+                       Hv, BF, st), n * (2 * 2 + 2 * 4)),
+        "gates_bwd": (("macai_gdr_gates_bwd", *gates_in, None, None, n, Hv, BF, st), n * (2 * 2 + 2 * 4 + 2 * 2)),
+        "gates_bwd_params": (("macai_gdr_gates_bwd_typed", *gates_in, P(part), P(dA), BF, P(ddt), BF, n, Hv, BF, st),
+                             n * (2 * 2 + 2 * 4 + 2 * 2) + 2 * part.numel() * 8),
     }
 
     def timed(fn):
@@ -481,7 +488,7 @@ def bench_producers(cfg, reps=20):
         e1.synchronize()
         return e0.elapsed_time(e1) / reps * 1e-3
 
-    wt = w4.to(bf).reshape(C, 1, 4)
+    wt = w4.reshape(C, 1, 4)
 
     def torch_conv():
         y = torch.nn.functional.silu(torch.nn.functional.conv1d(x.transpose(1, 2), wt, padding=3, groups=C)[..., :T])
