@@ -143,8 +143,8 @@ int macai_gdr_chunk_bwd(const void* q, const void* k, const void* v, const float
 
 /* The same with the gradients of a key head's value heads summed in the kernel: dq, dk [B, T, Hk, DK], the bits of
  * macai_gdr_chunk_bwd followed by macai_gdr_group_sum on each, without their per-head arrays and launches.  Taken where
- * macai_gdr_chunk_bwd_folds returns 1 for the shape on the current device (bf16, two value heads a key head, DK = DV and
- * more chunk-heads than the device runs at once, in whole pairs); EUNSUP elsewhere. */
+ * macai_gdr_chunk_bwd_folds returns 1 for the shape on the current device (bf16, two value heads a key head, DK = DV
+ * of 32, 64 or 128 and more chunk-heads than the device runs at once, in whole pairs); EUNSUP elsewhere. */
 int macai_gdr_chunk_bwd_folds(int64_t B, int64_t T, int64_t H, int64_t Hk, int64_t DK, int64_t DV, int32_t dtype,
                               const int32_t* pack, int64_t NT);
 int macai_gdr_chunk_bwd_folded(const void* q, const void* k, const void* v, const float* g, const float* beta,

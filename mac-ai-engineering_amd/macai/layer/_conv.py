@@ -56,7 +56,7 @@ DTYPES = (torch.float32, torch.bfloat16, torch.float16)
 def _unfit(x, w, kd: int, dk: int, rep: int, dv: int):
     """Why the convolution path cannot take these arguments, or None: x [B, T, C] in one of DTYPES with C = 2 kd +
     value_dim, w of C x 4 taps, kd a whole number of key heads of dk and value_dim of value heads of dv, each value head
-    group rep value heads a key head, every width a multiple of 8 (the kernels move 16-byte channel vectors)."""
+    group rep value heads a key head, every width a multiple of 8 (a lane's channel vector never crosses a head)."""
     if not isinstance(x, torch.Tensor) or not isinstance(w, torch.Tensor):
         return "x and the weight must be tensors"
     if x.dim() != 3:

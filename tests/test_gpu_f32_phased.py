@@ -1,6 +1,6 @@
 """The float32 state passes at key heads of 128, whose tiles fit LDS once only: refilled tile by tile between the groups
-of products on the two-wave form (value splits 4 and 8), all at once between chunks on the one-wave form (splits 1 and
-2).  One chunk, two, the last one a single token, and packed rows with one-token and empty sequences: the same bits."""
+of products on the two-wave form (the output pass at value splits 4 and 8, the reverse pass at 8 only, of one column
+slice), all at once between chunks elsewhere (splits 1 and 2, the reverse pass at 4).  One chunk, two, the last one a single token, and packed rows with one-token and empty sequences: the same bits."""
 import pytest
 import torch
 
