@@ -12,8 +12,8 @@
 // from du's windows (one writer an element) and the taps' gradient's sums over its steps; a tile of 64 rows adds its
 // blocks' sums in order through LDS, sum_columns_kernel the tiles' partials in tile order: deterministic.
 // The gates are one pass each way, an element a lane; over many rows the backward's also forms its workgroups' sums of
-// A_log's and dt_bias's gradients, which a second launch adds in a fixed order, over few a second pass takes a workgroup a
-// head (gate_direct_rows).
+// A_log's and dt_bias's gradients, which a second launch adds in a fixed order, over few a second pass takes a workgroup
+// a head (gate_direct_rows).
 #include <hip/hip_runtime.h>
 
 #include "gdr_abi.h"
@@ -473,8 +473,10 @@ __global__ void __launch_bounds__(CV_FEW_WIDE * (CV_ROWS / CV_FEW_STEPS)) conv_b
     for (int j = 0; j < CV_TAPS; ++j) mask(end + block - CV_HALO + j, ex[j]);
     mask(end + block, eg);
 #pragma unroll
-    for (int i = 0; i < VE; ++i)
-      head[BLOCKS][block][vec][i] = silu_grad<EXACT>(tap_dot<EXACT, VE>(tw, i, ex[0][i], ex[1][i], ex[2][i], ex[3][i]), eg[i]);
+    for (int i = 0; i < VE; ++i) {
+      const float u = tap_dot<EXACT, VE>(tw, i, ex[0][i], ex[1][i], ex[2][i], ex[3][i]);
+      head[BLOCKS][block][vec][i] = silu_grad<EXACT>(u, eg[i]);
+    }
   }
   if constexpr (TAPS) {
 #pragma unroll
@@ -519,8 +521,8 @@ __device__ __forceinline__ float load_code(const void* p, int t, size_t i) {
 }
 
 // out[i] = the sum over rows p = 0 .. P - 1 of in[p * n + i], in double, rounded to float32 and then to the type of code
-// ot: the fixed-order second stage of the taps' gradient.  A workgroup takes 64 outputs; each of its waves sums a quarter of the rows in row order, eight
-// rows' loads in flight together, and the quarters add in order.
+// ot: the fixed-order second stage of the taps' gradient.  A workgroup takes 64 outputs; each of its waves sums a quarter
+// of the rows in row order, eight rows' loads in flight together, and the quarters add in order.
 __global__ void __launch_bounds__(256) sum_columns_kernel(const float* in, void* out, int ot, int P, int n) {
   __shared__ double quarter[4][64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
@@ -728,9 +730,9 @@ int check_conv(const char* what, int64_t B, int64_t T, int64_t C, int64_t KD, in
 
 // Up to this many rows the parameters' gradients come from gates_params_direct_kernel (a workgroup a head), whose
 // chain is then the shorter one; past them from gates_bwd_sums_kernel and gates_params_kernel.  Where the two cross, with
-// the pass over the elements in each: at 8 to 64 heads 500 to 650 rows (16 heads: 5.7 against 6.2 us at 64, 7.6 against 6.4
-// at 1,024, 14.6 against 7.6 at 4,096).  Few heads make the sums' LDS chain of 256 / H rows long: 1 head crosses at 2,050
-// rows, 2 at 1,050, 3 to 7 at 500 to 750.  Many spread the direct form over the chip: 65 cross at 2,050, 96 and 128 at
+// the pass over the elements in each: at 8 to 64 heads 500 to 650 rows (16 heads: 5.7 against 6.2 us at 64, 7.6 against
+// 6.4 at 1,024, 14.6 against 7.6 at 4,096).  Few heads make the sums' LDS chain of 256 / H rows long: 1 head crosses at
+// 2,050 rows, 2 at 1,050, 3 to 7 at 500 to 750.  Many spread the direct form over the chip: 65 cross at 2,050, 96 and 128 at
 // 2,600, 192 and 256 at 2,900 to 3,300, more than 256 between 2,500 and 4,100.
 int64_t gate_direct_rows(int64_t H) {
   if (H <= 2) return 2048 / H;
@@ -800,8 +802,8 @@ int macai_gdr_conv_fwd_typed(const void* x, const void* w, int32_t wdtype, float
   ConvArgs a{x, w, taps, q, k, v, nullptr, nullptr, nullptr, nullptr, nullptr, (int)B, (int)T, (int)C, (int)KD, (int)DK,
              (int)REP, (int)conv_tiles(T)};
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)((C + 64 * CV_VE - 1) / (64 * CV_VE)), (unsigned)((T + 4 * CV_FWD_STEPS - 1) / (4 * CV_FWD_STEPS)),
-                  (unsigned)B);
+  const int64_t steps = 4 * CV_FWD_STEPS, span = 64 * CV_VE;
+  const dim3 grid((unsigned)((C + span - 1) / span), (unsigned)((T + steps - 1) / steps), (unsigned)B);
   DISPATCH_PT(dtype, DISPATCH_PV(vdtype, DISPATCH_PW(wdtype, hipLaunchKernelGGL((conv_fwd_kernel<PT, PV, PW>), grid,
                                                                                 dim3(256), 0, st, a))))
   return launched(what);
